@@ -1081,6 +1081,15 @@ int LaunchCore(const GemmCore &core, const EpiExtras &x, const void *a, const vo
         fast8 = fast8 && vec8(bias, core.Bias);
     }
     ep.fast8 = fast8 ? 1 : 0;
+    // The generic epilogue's runs of 8 columns need contiguous rows at any alignment, one of the five activations it
+    // compiles, and a float sum (the int32 accumulators have an epilogue of their own).
+    const bool act8 = x.act == KUDNN_ACT_UNIMPLEMENTED || x.act == KUDNN_ACT_RELU || x.act == KUDNN_ACT_SWISH ||
+                      x.act == KUDNN_ACT_GELU_TANH || x.act == KUDNN_ACT_GELU_ERF;
+    ep.vec8 = act8 && !ep.acc_i32 && Y.sn == 1 && (!x.hasSrc || x.Src.sn == 1) &&
+                      (!(x.storeC || beta != 0.0f) || core.C.sn == 1) &&
+                      (!core.hasBias || core.Bias.sn == 0 || core.Bias.sn == 1)
+                  ? 1
+                  : 0;
 
     int lrc = 0;
     if (core.engine == ENGINE_SKINNY_BF16) {

@@ -513,100 +513,118 @@ __device__ __forceinline__ void epi_apply4(const EpiParams &e, const EpiBatch &o
     epi_apply4_pre(e, ob, m, n, N, acc, epi_prefetch4(e, ob, m, n, N));
 }
 
-// Epilogue for eight consecutive columns n..n+7 of row m (n a multiple of 8): one 16-byte bf16 (or two
-// 16-byte f32) store per call when the output rows are contiguous and 8-element aligned (fast8).
-__device__ __forceinline__ void epi_apply8(const EpiParams &e, const EpiBatch &ob, int64_t m, int64_t n, int64_t N,
-                                           const float acc[8])
+// 8 consecutive elements of dtype dt as f32, from any element-aligned address (gfx950 serves vector accesses at any
+// alignment; a row of an odd number of elements makes every second one misaligned).
+template <typename E>
+struct __attribute__((packed, aligned(alignof(E)))) Run8 {
+    E v[8];
+};
+
+__device__ __forceinline__ void load_run8(const void *p, int dt, int64_t idx, float v[8])
 {
-    if (n + 7 < N && e.fast8) {
-        float v[8];
-        float bv[8];
-        if (e.bias != nullptr) {
-            const int64_t bi = ob.bias + m * e.bias_sm + n * e.bias_sn;
-            if (e.bias_sn == 0) {
-                const float b0 = load_elem(e.bias, e.bias_dt, bi);
+    if (dt == KUDNN_DT_BF16) {
+        const auto r = *reinterpret_cast<const Run8<uint16_t> *>(static_cast<const uint16_t *>(p) + idx);
 #pragma unroll
-                for (int q = 0; q < 8; ++q) bv[q] = b0;
-            } else if (e.bias_dt == KUDNN_DT_BF16) {
-                const uint4 raw = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(e.bias) + bi);
-                const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+        for (int q = 0; q < 8; ++q) v[q] = bf16_to_f32(r.v[q]);
+    } else if (dt == KUDNN_DT_F16) {
+        const auto r = *reinterpret_cast<const Run8<uint16_t> *>(static_cast<const uint16_t *>(p) + idx);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    bv[2 * q] = u2f(w[q] << 16);
-                    bv[2 * q + 1] = u2f(w[q] & 0xffff0000u);
-                }
+        for (int q = 0; q < 8; ++q) v[q] = f16_to_f32(r.v[q]);
+    } else if (dt == KUDNN_DT_F32) {
+        const auto r = *reinterpret_cast<const Run8<float> *>(static_cast<const float *>(p) + idx);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = r.v[q];
+    } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = load_elem(p, dt, idx + q);
+    }
+}
+
+// Stores 8 values rounded to dt as store_elem does.
+__device__ __forceinline__ void store_run8(void *p, int dt, int64_t idx, const float v[8])
+{
+    if (dt == KUDNN_DT_BF16 || dt == KUDNN_DT_F16) {
+        Run8<uint16_t> r;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) r.v[q] = dt == KUDNN_DT_BF16 ? f32_to_bf16_rne(v[q]) : f32_to_f16_rne(v[q]);
+        *reinterpret_cast<Run8<uint16_t> *>(static_cast<uint16_t *>(p) + idx) = r;
+    } else if (dt == KUDNN_DT_F32) {
+        Run8<float> r;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) r.v[q] = v[q];
+        *reinterpret_cast<Run8<float> *>(static_cast<float *>(p) + idx) = r;
+    } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) store_elem(p, dt, idx + q, v[q]);
+    }
+}
+
+// The generic epilogue of eight consecutive columns n .. n+7 of row m, all in bounds, with vec8 set by the host: the
+// tensor types are read at run time, every tensor is contiguous along n, at any alignment, and the activation is one
+// of the five compiled ones. The arithmetic and rounding of epi_apply. It serves what the fixed forms below do not: a
+// bias of another type than the output (Gemm's f32 bias on a 16-bit product), C stored beside linearRes, beta, rows of
+// an odd number of elements. Element by element, 2 bytes a store, this epilogue took longer than the products of a
+// short K: 4096 x 3520 x 1520 f16 with an f32 bias 141 us a call, 78 in runs of 8; 693 x 9704 x 5248 f16 with C stored
+// 225 and 139 us; 2112 x 2816 x 1094 bf16 120 and 55 us.
+__device__ __forceinline__ void epi_apply8(const EpiParams &e, const EpiBatch &ob, int64_t m, int64_t n, const float acc[8])
+{
+    float v[8], t[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = acc[q] * e.alpha;
+    if (e.beta != 0.0f) {
+        load_run8(e.c, e.c_dt, ob.c + m * e.c_sm + n, t);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] += e.beta * t[q];
+    }
+    if (e.bias != nullptr) {
+        const int64_t bi = ob.bias + m * e.bias_sm + n * e.bias_sn;
+        if (e.bias_sn == 0) {
+            const float b0 = load_elem(e.bias, e.bias_dt, bi);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) t[q] = b0;
+        } else {
+            load_run8(e.bias, e.bias_dt, bi, t);
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] += t[q];
+    }
+    if (e.c_dt == KUDNN_DT_BF16) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) round_bf16_pair(v[2 * q], v[2 * q + 1]);
+    } else if (e.c_dt == KUDNN_DT_F16) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = f16_to_f32(f32_to_f16_rne(v[q]));
+    }
+    if (e.store_c) {
+        store_run8(e.c, e.c_dt, ob.c + m * e.c_sm + n, v);
+    }
+    if (e.act != KUDNN_ACT_UNIMPLEMENTED) {
+        if (e.act == KUDNN_ACT_RELU) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = act_round(e.c_dt, KUDNN_ACT_RELU, act_relu(v[q], e.act_alpha));
+        } else {
+            if (e.act == KUDNN_ACT_SWISH) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[q] = act_swish(v[q], e.act_alpha);
+            } else if (e.act == KUDNN_ACT_GELU_TANH) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[q] = act_gelu_tanh(v[q]);
             } else {
 #pragma unroll
-                for (int q = 0; q < 8; ++q) bv[q] = load_elem(e.bias, e.bias_dt, bi + q);
+                for (int q = 0; q < 8; ++q) v[q] = act_gelu_erf(v[q]);
             }
-        } else {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) bv[q] = 0.0f;
+            for (int q = 0; q < 8; ++q) v[q] = act_round(e.c_dt, KUDNN_ACT_SWISH, v[q]);  // the three round alike
         }
+    }
+    if (e.bin != KUDNN_BINARY_NONE) {
+        load_run8(e.src, e.src_dt, ob.src + m * e.src_sm + n, t);
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            v[q] = round_store(e.c_dt, acc[q] * e.alpha + bv[q]);
+            v[q] = e.bin == KUDNN_BINARY_ADD ? v[q] + t[q] : (e.bin == KUDNN_BINARY_EXT ? fmaf(t[q], e.gamma, v[q]) : v[q] * t[q]);
         }
-        if (e.store_c) {
-            const int64_t ci = ob.c + m * e.c_sm + n;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) store_elem(e.c, e.c_dt, ci + q, v[q]);
-        }
-        if (e.act != KUDNN_ACT_UNIMPLEMENTED) {
-#pragma unroll
-            for (int q = 0; q < 8; ++q) v[q] = act_round(e.c_dt, e.act, apply_act(e.act, v[q], e.act_alpha, e.act_beta));
-        }
-        if (e.bin != KUDNN_BINARY_NONE) {
-            const int64_t si = ob.src + m * e.src_sm + n;
-            float sv[8];
-            if (e.src_dt == KUDNN_DT_BF16) {
-                const uint4 raw = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(e.src) + si);
-                const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    sv[2 * q] = u2f(w[q] << 16);
-                    sv[2 * q + 1] = u2f(w[q] & 0xffff0000u);
-                }
-            } else if (e.src_dt == KUDNN_DT_F32) {
-                const float4 t0 = *reinterpret_cast<const float4 *>(static_cast<const float *>(e.src) + si);
-                const float4 t1 = *reinterpret_cast<const float4 *>(static_cast<const float *>(e.src) + si + 4);
-                sv[0] = t0.x; sv[1] = t0.y; sv[2] = t0.z; sv[3] = t0.w;
-                sv[4] = t1.x; sv[5] = t1.y; sv[6] = t1.z; sv[7] = t1.w;
-            } else {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) sv[q] = load_elem(e.src, e.src_dt, si + q);
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                if (e.bin == KUDNN_BINARY_ADD) {
-                    v[q] = v[q] + sv[q];
-                } else if (e.bin == KUDNN_BINARY_EXT) {
-                    v[q] = fmaf(sv[q], e.gamma, v[q]);
-                } else {
-                    v[q] = v[q] * sv[q];
-                }
-            }
-        }
-        const int64_t yi = ob.y + m * e.y_sm + n;
-        if (e.y_dt == KUDNN_DT_BF16) {
-            uint32_t w[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                w[q] = pack_bf16x2_rne(v[2 * q], v[2 * q + 1]);
-            }
-            *reinterpret_cast<uint4 *>(static_cast<uint16_t *>(e.y) + yi) = make_uint4(w[0], w[1], w[2], w[3]);
-        } else if (e.y_dt == KUDNN_DT_F32) {
-            float *yp = static_cast<float *>(e.y) + yi;
-            *reinterpret_cast<float4 *>(yp) = make_float4(v[0], v[1], v[2], v[3]);
-            *reinterpret_cast<float4 *>(yp + 4) = make_float4(v[4], v[5], v[6], v[7]);
-        } else {
-#pragma unroll
-            for (int q = 0; q < 8; ++q) store_elem(e.y, e.y_dt, yi + q, v[q]);
-        }
-        return;
     }
-    epi_apply4(e, ob, m, n, N, acc);
-    epi_apply4(e, ob, m, n + 4, N, acc + 4);
+    store_run8(e.y, e.y_dt, ob.y + m * e.y_sm + n, v);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -959,8 +977,27 @@ __device__ __forceinline__ uint32_t i32_bias(const EpiParams &e, const EpiBatch 
 __device__ __forceinline__ void epi_i32_8(const EpiParams &e, const EpiBatch &ob, int64_t m, int64_t n, const float acc[8])
 {
     uint32_t v[8];
+    if (e.bias == nullptr || (e.bias_dt == KUDNN_DT_S32 && e.bias_sn == 1)) {
+        // one add of everything that is the same along n, the vectors 32 bytes at a time
+        const uint32_t cm = static_cast<uint32_t>(e.corr_c) +
+                            (e.corr_m != nullptr ? static_cast<uint32_t>(e.corr_m[ob.corr_m + m]) : 0u);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = f2u(acc[q]) + i32_bias(e, ob, m, n + q);
+        for (int q = 0; q < 8; ++q) v[q] = f2u(acc[q]) + cm;
+        if (e.bias != nullptr) {
+            const auto b = *reinterpret_cast<const Run8<uint32_t> *>(static_cast<const uint32_t *>(e.bias) + ob.bias +
+                                                                     m * e.bias_sm + n);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] += b.v[q];
+        }
+        if (e.corr_n != nullptr) {
+            const auto c = *reinterpret_cast<const Run8<uint32_t> *>(e.corr_n + ob.corr_n + n);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] += c.v[q];
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = f2u(acc[q]) + i32_bias(e, ob, m, n + q);
+    }
     uint4 *y = reinterpret_cast<uint4 *>(static_cast<uint32_t *>(e.y) + ob.y + m * e.y_sm + n);
     y[0] = make_uint4(v[0], v[1], v[2], v[3]);
     y[1] = make_uint4(v[4], v[5], v[6], v[7]);

@@ -476,6 +476,13 @@ __global__ __launch_bounds__(WM *WN * 64, 1) void gemm_mfma_kernel(GemmOperands 
                     continue;
                 }
                 const float *src = stage + r * kStagePitch + col8;
+                if (ep.vec8 && n + 7 < N) {
+                    const float4 lo = *reinterpret_cast<const float4 *>(src);
+                    const float4 hi = *reinterpret_cast<const float4 *>(src + 4);
+                    const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                    epi_apply8(ep, ob, m, n, v);
+                    continue;
+                }
 #pragma unroll 1
                 for (int q = 0; q < 8; ++q) {
                     if (n + q < N) {

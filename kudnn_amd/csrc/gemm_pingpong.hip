@@ -321,33 +321,47 @@ __device__ __forceinline__ void epilogue_edge(const EpiParams &ep, const EpiBatc
     });
 }
 
-// Epilogue of any tile in the generic form: one element at a time through epi_apply (activation read at run time).
+// Epilogue of any tile in the generic form (activation and tensor types read at run time): runs of 8 columns where the
+// host allows it (vec8), else one element at a time. The strips are a rolled loop with one copy of the epilogue's code;
+// only the staging, which must name its accumulators, is unrolled.
 __device__ __forceinline__ void epilogue_generic(const EpiParams &ep, const EpiBatch &ob, const f32x16_t (&acc)[4][2],
                                                  float *stage, int lane, int64_t mW, int64_t nW, int64_t M, int64_t N)
 {
     const int lrow = lane & 31, lh = lane >> 5;
     const int col8 = (lane & 3) * 8, rl = lane >> 2;
     __syncthreads();  // every wave is done with the tile buffers that the staging area reuses
-    sfor<4>([&](auto jc) __attribute__((always_inline)) {
-        constexpr int j = decltype(jc)::value;
+#pragma unroll 1
+    for (int j = 0; j < 4; ++j) {
         const int64_t n = nW + j * 32 + col8;
-        stage_strip(acc[j], stage, lrow, lh);
+        sfor<4>([&](auto jc) __attribute__((always_inline)) {
+            if (j == decltype(jc)::value) {
+                stage_strip(acc[decltype(jc)::value], stage, lrow, lh);
+                // keeps the four branches apart: merged into one that indexes acc by j, the accumulators live in scratch
+                asm volatile("; strip %0" ::"i"(decltype(jc)::value));
+            }
+        });
         wave_sync();
 #pragma unroll 1
         for (int ps = 0; ps < 4; ++ps) {
             const int r = rl + ps * 16;
             const int64_t m = mW + r;
-            if (m < M) {
+            const float *src = stage + r * kPitch + col8;
+            if (m < M && ep.vec8 && n + 7 < N) {
+                const float4 lo = *reinterpret_cast<const float4 *>(src);
+                const float4 hi = *reinterpret_cast<const float4 *>(src + 4);
+                const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                epi_apply8(ep, ob, m, n, v);
+            } else if (m < M) {
 #pragma unroll 1
                 for (int q = 0; q < 8; ++q) {
                     if (n + q < N) {
-                        epi_apply(ep, ob, m, n + q, stage[r * kPitch + col8 + q]);
+                        epi_apply(ep, ob, m, n + q, src[q]);
                     }
                 }
             }
         }
         wave_sync();
-    });
+    }
 }
 
 // Epilogue of the integer form (s8 x s8 -> s32): the accumulators hold int32 bit patterns; y = acc + bias exactly.
@@ -1124,8 +1138,12 @@ __global__ __launch_bounds__(256) void slice_reduce_kernel(const float *slices, 
         v[0] = lo[0]; v[1] = lo[1]; v[2] = lo[2]; v[3] = lo[3];
         v[4] = hi[0]; v[5] = hi[1]; v[6] = hi[2]; v[7] = hi[3];
         if constexpr (FORM == EPI_FORM_GENERIC) {
+            if (ep.vec8) {
+                epi_apply8(ep, ob, m, n, v);
+            } else {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) epi_apply(ep, ob, m, n + q, v[q]);
+                for (int q = 0; q < 8; ++q) epi_apply(ep, ob, m, n + q, v[q]);
+            }
         } else {
             epi_fast8<ACT, FORM>(ep, ob, m, n, v, epi_prefetch8<FORM>(ep, ob, m, n));
         }
