@@ -542,6 +542,12 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         core.A.staticPack = core.B.staticPack = true;
     }
     core.kp = (core.K + bk - 1) / bk * bk;
+    // A 16-bit weight stored [K][N] that can be read in place where the kernel does (see below): N contiguous, whole
+    // 64-deep k-tiles, whole 16-byte chunks of columns, 16-byte aligned k-rows and batches.
+    const bool kmajor16 = lowp16 && core.B.dt == core.computeDt && core.B.s_r == 1 && core.B.s_k >= core.N &&
+                          core.B.s_k % 8 == 0 && core.B.bs[0] % 8 == 0 && core.B.bs[1] % 8 == 0 &&
+                          core.B.bs[2] % 8 == 0 && core.K % 64 == 0 && core.N % 8 == 0 &&
+                          !std::getenv("KUDNN_HIP_PACK_KMAJOR");
 
     // engine and tile configuration
     const int64_t batches = core.Batches();
@@ -585,6 +591,22 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
             const bool fourWave = batches == 1 && t256 >= 32 && t256 <= 64 && kt <= 64 && core.B.s_r != 1;
             core.cfg = (t256 >= 80 || tailSplit || slices) && !fourWave ? KUDNN_CFG_BF16_PINGPONG_256x256
                                                                         : KUDNN_CFG_BF16_128x128;
+            if (lowp16) {
+                // below 256 rows: tiles with K dealt to the waves, against the other choice's estimate (kudnn_wavek_rule)
+                const int64_t t128 = (core.M + 127) / 128 * ((core.N + 127) / 128) * batches;
+                const int S = kudnn_kslice_rule(core.M, core.N, kt, batches, core.computeDt);
+                double other = 1e30;
+                if (core.cfg == KUDNN_CFG_BF16_128x128 && t128 >= KUDNN_SPLIT_MAX_TILES) {
+                    other = static_cast<double>((t128 + 255) / 256) * (4.0 + 0.66 * static_cast<double>(kt));
+                } else if (core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256) {
+                    const double div = S >= 2 ? S : 1;
+                    other = 9.0 + 1.2 * static_cast<double>(kt) / div +
+                            (S >= 2 ? static_cast<double>(S * core.M * core.N) * 8.0 / 3.6e6 : 0.0);
+                }
+                if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, kmajor16, other)) {
+                    core.cfg = wk;
+                }
+            }
         }
     } else {
         core.engine = ENGINE_MFMA_F32;
@@ -614,6 +636,7 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         bool okBf16 = core.computeDt != KUDNN_DT_F32 &&
                       (((f == KUDNN_CFG_BF16_256x256 || f == KUDNN_CFG_BF16_256x128 || f == KUDNN_CFG_BF16_128x128 ||
                          f == KUDNN_CFG_BF16_PINGPONG_256x256) && mfmaOk) ||
+                       (kudnn_is_wavek(f) && mfmaOk && lowp16) ||
                        (f == KUDNN_CFG_SKINNY_BF16 && core.M >= 2 && core.M <= 16 && lowp16) ||
                        (f == KUDNN_CFG_GEMV_MULTI_BF16 && core.M >= 2 && core.M <= 8 && lowp16) ||
                        (f == KUDNN_CFG_GEMV_KSPLIT_BF16 && core.M >= 2 && core.M <= 16 && lowp16));
@@ -628,15 +651,26 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
     // A K-major weight (B stored [K][N], N contiguous: C5's W{1,K,N} ABC) is read in place by the ping-pong kernel,
     // through transposing LDS reads, instead of being packed on every run; it needs 64-deep k-tiles, N a multiple of
     // 8 (whole 16-byte column chunks; an edge tile's columns past N are computed and never stored), 16-byte aligned
-    // k-rows and batches, and 32-bit offsets.
-    const bool bBatchAligned = core.B.bs[0] % 8 == 0 && core.B.bs[1] % 8 == 0 && core.B.bs[2] % 8 == 0;
-    if (core.engine == ENGINE_MFMA_BF16 && core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256 &&
-        (core.computeDt == KUDNN_DT_BF16 || core.computeDt == KUDNN_DT_F16) && core.B.dt == core.computeDt &&
-        core.B.s_r == 1 && core.B.s_k >= core.N && core.B.s_k % 8 == 0 && bBatchAligned && core.K % 64 == 0 &&
-        core.N % 8 == 0 && core.K * core.B.s_k * 2 < (int64_t(1) << 31) &&
-        core.M * std::max<int64_t>(core.A.s_r, core.kp) * 2 < (int64_t(1) << 31) && !std::getenv("KUDNN_HIP_PACK_KMAJOR")) {
+    // k-rows and batches, and 32-bit offsets. The wave-K tiles of 64 and 128 columns do the same with 64-bit addresses.
+    const bool wavek = core.engine == ENGINE_MFMA_BF16 && kudnn_is_wavek(core.cfg);
+    const bool wide = core.cfg == KUDNN_CFG_WAVEK_32x64 || core.cfg == KUDNN_CFG_WAVEK_64x64 ||
+                      core.cfg == KUDNN_CFG_WAVEK_64x64_W4 || core.cfg == KUDNN_CFG_WAVEK_64x128;
+    if (kmajor16 && ((wavek && wide) ||
+                     (core.engine == ENGINE_MFMA_BF16 && core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256 &&
+                      core.K * core.B.s_k * 2 < (int64_t(1) << 31) &&
+                      core.M * std::max<int64_t>(core.A.s_r, core.kp) * 2 < (int64_t(1) << 31)))) {
         core.B.kmajor = true;
         core.B.staticPack = false;
+    }
+    // The wave-K kernel masks the K tail itself where both operands lie contiguous along K: whole 16-byte chunks do.
+    if (wavek && core.K % bk != 0) {
+        const auto direct = [&](const OperandSpec &o) {
+            return o.dt == core.computeDt && o.s_k == 1 && core.K % epc == 0 && o.s_r % epc == 0 && o.bs[0] % epc == 0 &&
+                   o.bs[1] % epc == 0 && o.bs[2] % epc == 0;
+        };
+        if (direct(core.A) && direct(core.B)) {
+            core.A.staticPack = core.B.staticPack = false;
+        }
     }
     // The same for an fp32 weight stored [K][N] (the reference's Matmul mode passes W in ABCDE,
     // matmul_gtest.cpp:248-257), read in place by the 4-wave fp32 kernels (128 x 128 and 64 x 64) and by the k-slice
@@ -661,6 +695,13 @@ const char *CfgName(int cfg)
         case KUDNN_CFG_BF16_256x128: return "mfma_bf16_256x128";
         case KUDNN_CFG_BF16_128x128: return "mfma_bf16_128x128";
         case KUDNN_CFG_BF16_PINGPONG_256x256: return "mfma_bf16_pingpong_256x256";
+        case KUDNN_CFG_WAVEK_32x16: return "mfma_bf16_wavek_32x16_w8";
+        case KUDNN_CFG_WAVEK_32x32: return "mfma_bf16_wavek_32x32_w8";
+        case KUDNN_CFG_WAVEK_32x64: return "mfma_bf16_wavek_32x64_w6";
+        case KUDNN_CFG_WAVEK_64x32: return "mfma_bf16_wavek_64x32_w6";
+        case KUDNN_CFG_WAVEK_64x64: return "mfma_bf16_wavek_64x64_w8";
+        case KUDNN_CFG_WAVEK_64x64_W4: return "mfma_bf16_wavek_64x64_w4";
+        case KUDNN_CFG_WAVEK_64x128: return "mfma_bf16_wavek_64x128_w4";
         case KUDNN_CFG_F32_128x128: return "mfma_f32_128x128";
         case KUDNN_CFG_F32_64x64: return "mfma_f32_64x64";
         case KUDNN_CFG_F32_KSLICE_16x32: return "mfma_f32_kslice_16x32";
@@ -898,8 +939,9 @@ int LaunchCore(const GemmCore &core, const EpiExtras &x, const void *a, const vo
     op.M = core.M;
     op.N = core.N;
     // MFMA kernels run whole k-tiles: when K is not a multiple of the tile both operands were packed with
-    // zero padding up to kp (and kp == K otherwise). The skinny kernel masks its own K tail.
-    op.K = core.engine == ENGINE_SKINNY_BF16 ? core.K : core.kp;
+    // zero padding up to kp (and kp == K otherwise). The skinny and wave-K kernels mask their own K tail.
+    const bool wavek = core.engine == ENGINE_MFMA_BF16 && kudnn_is_wavek(core.cfg);
+    op.K = core.engine == ENGINE_SKINNY_BF16 || wavek ? core.K : core.kp;
     auto setupOperand = [&](const OperandSpec &o, const void *ptr, bool pack, void *dst, const void *&outPtr,
                             int64_t &ld, int64_t outBs[3]) -> int {
         if (!pack) {
@@ -1095,7 +1137,9 @@ int LaunchCore(const GemmCore &core, const EpiExtras &x, const void *a, const vo
     if (core.engine == ENGINE_SKINNY_BF16) {
         lrc = kudnn_launch_skinny(op, ep, batches, core.computeDt, core.cfg, stream);
     } else if (core.engine == ENGINE_MFMA_BF16) {
-        if (core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256 && kudnn_pingpong_eligible(op, core.computeDt)) {
+        if (wavek) {
+            lrc = kudnn_launch_gemm_wavek(op, ep, batches, core.computeDt, core.cfg, stream);
+        } else if (core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256 && kudnn_pingpong_eligible(op, core.computeDt)) {
             lrc = kudnn_launch_gemm_pingpong(op, ep, batches, core.computeDt, tailWs, slicesOk, stream);
         } else if (op.b_kmajor) {
             // only the ping-pong kernel reads a K-major B (the plan's conditions make it eligible)

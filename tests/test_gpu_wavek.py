@@ -1,0 +1,113 @@
+"""The wave-K kernel (small tiles whose K is dealt to the workgroup's waves): every tile at the edges of M, N and K, both
+weight layouts, batches, graph replay and the planner's choices, against the oracle. Integer-valued inputs make the f32
+sums exact in any order, so the comparisons are bit for bit."""
+import numpy as np
+import pytest
+
+import kudnn_amd as K
+import oracle as O
+from support import Case, compare, explainer, from_device, zeros_device
+from test_gpu_layouts import T, run_gemm
+
+torch = pytest.importorskip("torch")
+
+TILES = {"30": "32x16_w8", "31": "32x32_w8", "32": "32x64_w6", "33": "64x32_w6", "34": "64x64_w8", "35": "64x64_w4",
+         "36": "64x128_w4"}
+WIDE = ("32", "34", "35", "36")  # the tiles that read a [K][N] weight in place
+
+
+@pytest.fixture
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    K.lib()
+
+
+# K: one chunk, one k-tile, a k-tile and a chunk, fewer k-tiles than waves, one each, one more; odd (packed)
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", list(TILES))
+@pytest.mark.parametrize("M,N,Kd", [(17, 16, 8), (32, 33, 64), (33, 130, 72), (64, 128, 320), (65, 264, 512), (70, 40, 584),
+                                    (255, 7, 1000), (40, 72, 131)])
+@pytest.mark.parametrize("dt", [O.BF16, O.F16])
+def test_tiles_exact(gpu, monkeypatch, cfg, M, N, Kd, dt):
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
+    d, _ = run_gemm(T([M, Kd], dt), T([Kd, N], dt, "BA"), T([M, N], dt), T([1, N], O.F32), seed=850, int_valued=True)
+    assert TILES[cfg] in d and ("pack" in d) == (Kd % 8 != 0), d
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", list(TILES))
+@pytest.mark.parametrize("M,N,Kd", [(17, 8, 64), (64, 128, 448), (70, 200, 512), (130, 264, 64), (33, 72, 200), (33, 70, 128)])
+def test_kmajor_weight_exact(gpu, monkeypatch, cfg, M, N, Kd):
+    # [K][N]: in place by the wide tiles when N is a multiple of 8 and K of 64, packed otherwise
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
+    d, _ = run_gemm(T([M, Kd], O.BF16), T([Kd, N], O.BF16, "AB"), T([M, N], O.F32), None, seed=851, int_valued=True)
+    assert ("kmajorB" in d) == (cfg in WIDE and N % 8 == 0 and Kd % 64 == 0), d
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", ["30", "35"])
+def test_batches_and_pitches_exact(gpu, monkeypatch, cfg):
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
+    run_gemm(T([3, 40, 136], O.BF16, "ABC", [40 * 144, 144, 1]), T([3, 136, 72], O.BF16, "ACB"), T([3, 40, 72], O.BF16),
+             T([3, 1, 72], O.F32), alpha=0.5, beta=0.5, seed=852, int_valued=True)
+    run_gemm(T([2, 3, 40, 128], O.F16), T([2, 1, 128, 72], O.F16), T([2, 3, 40, 72], O.F16), None, seed=853, int_valued=True)
+
+
+@pytest.mark.gpu
+def test_rows_past_k_stay_out(gpu, monkeypatch):
+    # the 16-byte chunks past K hold Inf and NaN (the next elements of a longer row): none may reach the sums
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", "34")
+    M, N, Kd, P = 40, 72, 200, 256
+    x = torch.full((M, P), float("nan"), device="cuda", dtype=torch.bfloat16)
+    w = torch.full((N, P), float("inf"), device="cuda", dtype=torch.bfloat16)
+    x[:, :Kd] = 1.0
+    w[:, :Kd] = 0.5
+    y = torch.zeros(M, N, device="cuda", dtype=torch.float32)
+    plan = K.Gemm(K.desc([M, Kd], K.BF16, "AB", [P, 1]), K.desc([Kd, N], K.BF16, "BA", [1, P]), K.desc([M, N], K.F32))
+    assert "wavek" in plan.describe() and "pack" not in plan.describe(), plan.describe()
+    plan.run(x, w, y)
+    torch.cuda.synchronize()
+    assert bool((y == 0.5 * Kd).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,Kd,wl", [(64, 1024, 2048, "BA"), (100, 600, 1096, "BA"), (64, 1024, 2048, "AB")])
+def test_planner_plans_and_graph_replays(gpu, M, N, Kd, wl):
+    dt = O.BF16
+    x = Case([M, Kd], dt, seed=860, dist="normal", lo=0.0, hi=1.0)
+    w = Case([Kd, N], dt, wl, seed=861, dist="normal", lo=0.0, hi=0.05)
+    s = Case([M, N], dt, seed=862, lo=-1.0, hi=1.0)
+    y = Case([M, N], dt, zero=True)
+    plan = K.LinearPostOps(x.desc, w.desc, y.desc, None, act=K.ACT_GELU_TANH, binary=K.BIN_ADD, src=s.desc)
+    assert "wavek" in plan.describe(), plan.describe()
+    dx, dw, ds, dy = x.device(), w.device(), s.device(), zeros_device(y)
+    plan.run(dx, dw, dy, None, ds)
+    torch.cuda.synchronize()
+    ref = y.clone_empty()
+    O.linear_postops(x.t, w.t, ref, None, O.ACT_GELU_TANH, 0.0, O.BIN_ADD, s.t)
+    eager = from_device(dy, dt)
+    why = explainer(dt, x.t, w.t, None, (M, N), act=K.ACT_GELU_TANH, binary=K.BIN_ADD, src=s.t)
+    compare(eager, ref.buf, dt, plan.describe(), explain=why)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        plan.run(dx, dw, dy, None, ds, stream=torch.cuda.current_stream())
+    for _ in range(3):
+        dy.zero_()
+        torch.randn(1 << 16, device="cuda").sum()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(from_device(dy, dt), eager)
+
+
+def test_planner_rule():
+    def plan(M, Kd, N, wl="BA", dt=K.BF16):
+        return K.LinearPostOps(K.desc([M, Kd], dt), K.desc([Kd, N], dt, wl), K.desc([M, N], dt)).describe()
+    assert plan(17, 4096, 4096).startswith("mfma_bf16_wavek_32x16")
+    assert plan(64, 4096, 4096, dt=K.F16).startswith("mfma_f16_wavek_32x32")
+    assert plan(64, 4096, 11008).startswith("mfma_bf16_wavek_64x64")
+    assert "kmajorB" in plan(64, 4096, 4096, "AB") and "packA packB" in plan(64, 1000, 4096, "AB")
+    assert "pack" not in plan(100, 1000, 4096) and "packA packB" in plan(100, 1001, 4096)
+    assert plan(16, 4096, 4096).startswith("skinny") and "wavek" not in plan(256, 4096, 4096)
+    assert "wavek" not in plan(255, 4096, 14336) and "wavek" not in plan(40, 128, 4096)
