@@ -549,6 +549,18 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
                           core.B.bs[2] % 8 == 0 && core.K % 64 == 0 && core.N % 8 == 0 &&
                           !std::getenv("KUDNN_HIP_PACK_KMAJOR");
 
+    // Whether the wave-K kernel can read both operands in place: contiguous along K in whole 16-byte chunks (it masks the
+    // K tail itself), of the compute type, a u8 A of an integer product, or an 8-bit weight of an f16 product.
+    const auto chunked = [&](const OperandSpec &o) {
+        const int64_t c = 16 / DtSize(o.dt);
+        return o.s_k == 1 && core.K % c == 0 && o.s_r % c == 0 && o.bs[0] % c == 0 && o.bs[1] % c == 0 && o.bs[2] % c == 0;
+    };
+    const bool inPlaceA = chunked(core.A) && (core.A.dt == core.computeDt ||
+                                              (core.computeDt == KUDNN_DT_S8 && core.A.dt == KUDNN_DT_U8));
+    const bool w8 = core.computeDt == KUDNN_DT_F16 && (core.B.dt == KUDNN_DT_S8 || core.B.dt == KUDNN_DT_U8);
+    const bool inPlaceAB = inPlaceA && chunked(core.B) && (core.B.dt == core.computeDt || w8);
+    const bool weight8 = w8 && inPlaceAB;
+
     // engine and tile configuration
     const int64_t batches = core.Batches();
     if (core.computeDt != KUDNN_DT_F32) {
@@ -591,21 +603,31 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
             const bool fourWave = batches == 1 && t256 >= 32 && t256 <= 64 && kt <= 64 && core.B.s_r != 1;
             core.cfg = (t256 >= 80 || tailSplit || slices) && !fourWave ? KUDNN_CFG_BF16_PINGPONG_256x256
                                                                         : KUDNN_CFG_BF16_128x128;
-            if (lowp16) {
-                // below 256 rows: tiles with K dealt to the waves, against the other choice's estimate (kudnn_wavek_rule)
-                const int64_t t128 = (core.M + 127) / 128 * ((core.N + 127) / 128) * batches;
-                const int S = kudnn_kslice_rule(core.M, core.N, kt, batches, core.computeDt);
-                double other = 1e30;
-                if (core.cfg == KUDNN_CFG_BF16_128x128 && t128 >= KUDNN_SPLIT_MAX_TILES) {
-                    other = static_cast<double>((t128 + 255) / 256) * (4.0 + 0.66 * static_cast<double>(kt));
-                } else if (core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256) {
-                    const double div = S >= 2 ? S : 1;
-                    other = 9.0 + 1.2 * static_cast<double>(kt) / div +
-                            (S >= 2 ? static_cast<double>(S * core.M * core.N) * 8.0 / 3.6e6 : 0.0);
-                }
-                if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, kmajor16, other)) {
-                    core.cfg = wk;
-                }
+        }
+        // Tiles with K dealt to the waves, where their estimate (kudnn_wavek_rule) beats this one of the choice above.
+        // The 4-wave kernel took 4 + 0.66 us per k-tile and round of 256 tiles (s8 0.72; 30 us and more where it splits
+        // K), the ping-pong kernel 5 + 1.15 us per k-tile and round, in S slices 9 + 1.2 us per k-tile of a slice + the
+        // sums' way at 3.6 TB/s; a u8 A adds two packs and the row sums of the weight, an 8-bit weight of an f16 product
+        // its pack.
+        const int64_t t128 = (core.M + 127) / 128 * ((core.N + 127) / 128) * batches;
+        const int64_t t256 = (core.M + 255) / 256 * ((core.N + 255) / 256) * batches;
+        const double kt = static_cast<double>(core.kp * DtSize(core.computeDt) / 128);
+        const double nk = static_cast<double>(core.N * core.K), mn = static_cast<double>(core.M * core.N);
+        const bool s8 = core.computeDt == KUDNN_DT_S8;
+        const int S = kudnn_kslice_rule(core.M, core.N, static_cast<int64_t>(kt), batches, core.computeDt);
+        double other = 1e30;
+        if (core.cfg == KUDNN_CFG_BF16_128x128 && (s8 || t128 >= KUDNN_SPLIT_MAX_TILES)) {
+            other = static_cast<double>((t128 + 255) / 256) * (4.0 + (s8 ? 0.72 : 0.66) * kt);
+        } else if (core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256) {
+            other = S >= 2 ? 9.0 + 1.2 * kt / S + S * mn * 8.0 / 3.6e6 : 5.0 + 1.15 * kt * static_cast<double>((t256 + 255) / 256);
+        }
+        other += weight8 ? 3.0 + nk * 0.75e-6 : (s8 && core.A.dt == KUDNN_DT_U8 ? 14.0 + nk * 0.47e-6 : 0.0);
+        // an integer product with a u8 weight needs row sums of A, and an 8-bit weight of an f16 product that cannot be
+        // read in place is packed to f16: both stay with the other kernels
+        if (core.B.dt != KUDNN_DT_U8 || weight8) {
+            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, core.computeDt, weight8, kmajor16, other)) {
+                core.engine = ENGINE_MFMA_BF16;
+                core.cfg = wk;
             }
         }
     } else {
@@ -636,7 +658,7 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         bool okBf16 = core.computeDt != KUDNN_DT_F32 &&
                       (((f == KUDNN_CFG_BF16_256x256 || f == KUDNN_CFG_BF16_256x128 || f == KUDNN_CFG_BF16_128x128 ||
                          f == KUDNN_CFG_BF16_PINGPONG_256x256) && mfmaOk) ||
-                       (kudnn_is_wavek(f) && mfmaOk && lowp16) ||
+                       (kudnn_is_wavek(f) && (lowp16 || core.B.dt == KUDNN_DT_S8)) ||
                        (f == KUDNN_CFG_SKINNY_BF16 && core.M >= 2 && core.M <= 16 && lowp16) ||
                        (f == KUDNN_CFG_GEMV_MULTI_BF16 && core.M >= 2 && core.M <= 8 && lowp16) ||
                        (f == KUDNN_CFG_GEMV_KSPLIT_BF16 && core.M >= 2 && core.M <= 16 && lowp16));
@@ -662,15 +684,8 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         core.B.kmajor = true;
         core.B.staticPack = false;
     }
-    // The wave-K kernel masks the K tail itself where both operands lie contiguous along K: whole 16-byte chunks do.
-    if (wavek && core.K % bk != 0) {
-        const auto direct = [&](const OperandSpec &o) {
-            return o.dt == core.computeDt && o.s_k == 1 && core.K % epc == 0 && o.s_r % epc == 0 && o.bs[0] % epc == 0 &&
-                   o.bs[1] % epc == 0 && o.bs[2] % epc == 0;
-        };
-        if (direct(core.A) && direct(core.B)) {
-            core.A.staticPack = core.B.staticPack = false;
-        }
+    if (wavek && !core.B.kmajor && inPlaceAB) {
+        core.A.staticPack = core.B.staticPack = false;
     }
     // The same for an fp32 weight stored [K][N] (the reference's Matmul mode passes W in ABCDE,
     // matmul_gtest.cpp:248-257), read in place by the 4-wave fp32 kernels (128 x 128 and 64 x 64) and by the k-slice
@@ -695,12 +710,14 @@ const char *CfgName(int cfg)
         case KUDNN_CFG_BF16_256x128: return "mfma_bf16_256x128";
         case KUDNN_CFG_BF16_128x128: return "mfma_bf16_128x128";
         case KUDNN_CFG_BF16_PINGPONG_256x256: return "mfma_bf16_pingpong_256x256";
+        case KUDNN_CFG_WAVEK_16x16: return "mfma_bf16_wavek_16x16_w8";
+        case KUDNN_CFG_WAVEK_16x32: return "mfma_bf16_wavek_16x32_w8";
         case KUDNN_CFG_WAVEK_32x16: return "mfma_bf16_wavek_32x16_w8";
         case KUDNN_CFG_WAVEK_32x32: return "mfma_bf16_wavek_32x32_w8";
         case KUDNN_CFG_WAVEK_32x64: return "mfma_bf16_wavek_32x64_w6";
         case KUDNN_CFG_WAVEK_64x32: return "mfma_bf16_wavek_64x32_w6";
-        case KUDNN_CFG_WAVEK_64x64: return "mfma_bf16_wavek_64x64_w8";
-        case KUDNN_CFG_WAVEK_64x64_W4: return "mfma_bf16_wavek_64x64_w4";
+        case KUDNN_CFG_WAVEK_64x64: return "mfma_bf16_wavek_64x64";
+        case KUDNN_CFG_WAVEK_64x64_W4: return "mfma_bf16_wavek_64x64_2percu";
         case KUDNN_CFG_WAVEK_64x128: return "mfma_bf16_wavek_64x128_w4";
         case KUDNN_CFG_F32_128x128: return "mfma_f32_128x128";
         case KUDNN_CFG_F32_64x64: return "mfma_f32_64x64";
@@ -1006,8 +1023,8 @@ int LaunchCore(const GemmCore &core, const EpiExtras &x, const void *a, const vo
     const bool aU8 = core.computeDt == KUDNN_DT_S8 && core.A.dt == KUDNN_DT_U8;
     const bool bU8 = core.computeDt == KUDNN_DT_S8 && core.B.dt == KUDNN_DT_U8;
     const int64_t copiesA = allBroadcast(core.A) ? 1 : batches, copiesB = allBroadcast(core.B) ? 1 : batches;
-    const size_t wsCm = bU8 ? align256(static_cast<size_t>(copiesA * core.M) * sizeof(int32_t)) : 0;
-    const size_t wsCn = aU8 ? align256(static_cast<size_t>(copiesB * core.N) * sizeof(int32_t)) : 0;
+    const size_t wsCm = bU8 && !wavek ? align256(static_cast<size_t>(copiesA * core.M) * sizeof(int32_t)) : 0;
+    const size_t wsCn = aU8 && !wavek ? align256(static_cast<size_t>(copiesB * core.N) * sizeof(int32_t)) : 0;
     uint32_t *counters = nullptr;
     if (wsA + wsB + wsS + wsK + wsCm + wsCn > 0) {
         int arc = KUDNN_STATUS_SUCCESS;
@@ -1138,7 +1155,10 @@ int LaunchCore(const GemmCore &core, const EpiExtras &x, const void *a, const vo
         lrc = kudnn_launch_skinny(op, ep, batches, core.computeDt, core.cfg, stream);
     } else if (core.engine == ENGINE_MFMA_BF16) {
         if (wavek) {
-            lrc = kudnn_launch_gemm_wavek(op, ep, batches, core.computeDt, core.cfg, stream);
+            // the weight's type as the kernel finds it; u8 under s8 stands for a u8 A
+            const int bt = core.computeDt == KUDNN_DT_S8 ? core.A.dt : (packB ? core.computeDt : core.B.dt);
+            op.a_u8 = aU8 && !packA ? 1 : 0;
+            lrc = kudnn_launch_gemm_wavek(op, ep, batches, core.computeDt, bt, core.cfg, stream);
         } else if (core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256 && kudnn_pingpong_eligible(op, core.computeDt)) {
             lrc = kudnn_launch_gemm_pingpong(op, ep, batches, core.computeDt, tailWs, slicesOk, stream);
         } else if (op.b_kmajor) {

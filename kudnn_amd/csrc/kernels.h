@@ -19,16 +19,18 @@ enum {
     KUDNN_CFG_GEMV_BF16 = 21,  // M == 1: one wave per weight row, X staged in LDS (skinny engine)
     KUDNN_CFG_GEMV_MULTI_BF16 = 22,  // 2 <= M <= 5 (M <= 8 forced): one wave per weight row, X staged in LDS
     KUDNN_CFG_GEMV_KSPLIT_BF16 = 23,  // 2 <= M <= 16, K <= 4096, one batch: K split over 8 waves, X in registers
-    // 16 < M < 256, 16-bit: a small tile per workgroup, its K dealt to the waves (gemm_wavek.hip); tile x waves
-    KUDNN_CFG_WAVEK_32x16 = 30,    // 8 waves
+    // a small tile per workgroup, its K dealt to the waves (gemm_wavek.hip, kudnn_wavek_rule)
+    KUDNN_CFG_WAVEK_16x16 = 28,    // 8 waves; 8-bit weights
+    KUDNN_CFG_WAVEK_16x32 = 29,    // 8; 8-bit weights
+    KUDNN_CFG_WAVEK_32x16 = 30,    // 8
     KUDNN_CFG_WAVEK_32x32 = 31,    // 8
     KUDNN_CFG_WAVEK_32x64 = 32,    // 6
     KUDNN_CFG_WAVEK_64x32 = 33,    // 6
-    KUDNN_CFG_WAVEK_64x64 = 34,    // 8
-    KUDNN_CFG_WAVEK_64x64_W4 = 35, // 4
+    KUDNN_CFG_WAVEK_64x64 = 34,    // 8 (8-bit weights of f16: 6)
+    KUDNN_CFG_WAVEK_64x64_W4 = 35, // 4 (8-bit weights of f16: 3)
     KUDNN_CFG_WAVEK_64x128 = 36,   // 4
 };
-inline bool kudnn_is_wavek(int cfg) { return cfg >= KUDNN_CFG_WAVEK_32x16 && cfg <= KUDNN_CFG_WAVEK_64x128; }
+inline bool kudnn_is_wavek(int cfg) { return cfg >= KUDNN_CFG_WAVEK_16x16 && cfg <= KUDNN_CFG_WAVEK_64x128; }
 
 // Returns 0 on success, -1 if the launch failed or cfg is unknown. `ct` is the operand (compute) type of the 16- and
 // 8-bit kernels: KUDNN_DT_BF16, KUDNN_DT_F16 (f32 accumulation) or KUDNN_DT_S8 (int32 accumulation, integer
@@ -103,48 +105,61 @@ inline int kudnn_tail_slice_rule(int64_t M, int64_t N, int64_t KT, int64_t batch
     return S >= 2 ? static_cast<int>(S) : 0;
 }
 
-// Tiles whose K is dealt to the workgroup's waves (gemm_wavek.hip): bf16 / f16, 16-byte aligned rows and bases; op.K is
-// the true K (a multiple of 8, or rows packed with zeros up to whole chunks); b_kmajor with N and ldb multiples of 8 and
-// the tiles of 64 or 128 columns. No workspace.
-int kudnn_launch_gemm_wavek(const GemmOperands &op, const EpiParams &ep, int64_t batches, int ct, int cfg,
+// Tiles whose K is dealt to the workgroup's waves (gemm_wavek.hip): 16-byte aligned rows and bases; op.K is the true K
+// (whole 16-byte chunks, or rows packed with zeros up to whole chunks); b_kmajor (16-bit) with N and ldb multiples of 8
+// and the tiles of 64 or 128 columns. `bt` is the weight's stored type: ct, s8 or u8 under f16, and u8 under s8 for a u8
+// A beside an s8 weight (the term of the -128 shift is added here; op.a_u8 says whether A still has to be shifted). No
+// workspace.
+int kudnn_launch_gemm_wavek(const GemmOperands &op, const EpiParams &ep, int64_t batches, int ct, int bt, int cfg,
                             hipStream_t stream);
 
-// The wave-K tile for a 16-bit product of 16 < M < 256 rows (0: the kernel the other rules chose). The estimate is what
-// the measurements of 7 tiles over M = 17..512 and N, K = 2048..14336 (bf16, weights rotated past the Infinity Cache)
-// fit: 4.2 us a call, plus the larger of the weight's stream from HBM at 6.6 TB/s and the busiest CU's copies, nsPerKB
-// per KB of A and B (a tenth more when more tiles come to a CU than fit beside one another), plus a part of the smaller.
-// Over 26 drawn shapes the choice was within 7 % of the best tile but for 3 (19 %). otherUs is the same kind of estimate
-// for the other rules' kernel: the 4-wave kernel of 128 x 128 tiles took 4 + 0.66 us per k-tile and round where it does
-// not split K, the ping-pong kernel in S slices 9 + 1.2 us per k-tile of a slice + the sums' way at 3.6 TB/s.
-// 64 x 4096 x 4096: 10 us against 31; 64 x 11008 x 4096: 22 against 48; 192 x 4096 x 11008: 45 against 48; at
-// 255 x 14336 x 4096 (55 against 47) and 160 x 14336 x 2048 (32 against 28) the 4-wave kernel stays. From 256 rows on
-// the tiles re-read A and B too often for a weight's whole width (512 x 11008 x 4096: 83 against 76).
-inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, bool kmajor, double otherUs)
+// The wave-K tile for a product (0: the kernel the other rules chose). The estimate is what the measurements of 7 tiles
+// over M = 17..1030 and N, K = 2048..14336 (weights rotated past the Infinity Cache) fit: 4.2 us a call, plus the largest
+// of the weight's stream from HBM at 6.6 TB/s, the busiest CU's copies, nsPerKB per KB of A and B (`over` times that when
+// more tiles come to a CU than fit beside one another), and the products at 0.8 PFLOP/s (8-bit: 1.4), plus a part of the
+// stream. Over 26 drawn bf16 shapes the choice was within 7 % of the best tile but for 3 (19 %). otherUs is the same kind
+// of estimate for the other rules' kernel (BuildCore). Measured, against the other kernel: bf16 64 x 4096 x 4096 10 us (31),
+// 64 x 11008 x 4096 22 (48), 192 x 4096 x 11008 45 (48), 400 x 4096 x 4096 27 (45); f16 x s8 4 x 4096 x 4096 6.1 (21.5),
+// 128 x 4096 x 4096 12 (55); u8 x s8 64 x 4096 x 4096 7.5 (47), 1024 x 4096 x 4096 40 (51). The others stay where a weight
+// is wide for its depth (bf16 255 x 14336 x 4096 55 against 47, 160 x 14336 x 2048 32 against 28) and where M is large:
+// the small tiles then re-read A and B too often. 16-bit products of up to 16 rows have the decode kernels; those of
+// 256 rows or more in whole 128-row tiles keep the plans that the dispatch sweep fixed for them. Less than 4 whole
+// k-tiles leave most waves without one.
+inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, int ct, bool weight8, bool kmajor,
+                            double otherUs)
 {
     struct Tile {
-        int cfg, bm, bn, waves, fit;
-        double nsPerKB;
+        int cfg, bm, bn, waves;
+        double nsPerKB, over;
     };
-    static const Tile kTiles[] = {{KUDNN_CFG_WAVEK_32x16, 32, 16, 8, 3, 11.5}, {KUDNN_CFG_WAVEK_32x32, 32, 32, 8, 2, 11.7},
-                                  {KUDNN_CFG_WAVEK_64x32, 64, 32, 6, 2, 11.3}, {KUDNN_CFG_WAVEK_32x64, 32, 64, 6, 2, 11.8},
-                                  {KUDNN_CFG_WAVEK_64x64, 64, 64, 8, 1, 12.6}, {KUDNN_CFG_WAVEK_64x64_W4, 64, 64, 4, 2, 12.9},
-                                  {KUDNN_CFG_WAVEK_64x128, 64, 128, 4, 1, 15.5}};
-    const int64_t KT = (K + 63) / 64;
-    if (M <= 16 || M >= 256 || KT < 4) {
+    static const Tile kTiles[] = {{KUDNN_CFG_WAVEK_16x16, 16, 16, 8, 11.5, 1.1}, {KUDNN_CFG_WAVEK_16x32, 16, 32, 8, 11.6, 1.1},
+                                  {KUDNN_CFG_WAVEK_32x16, 32, 16, 8, 11.5, 1.1}, {KUDNN_CFG_WAVEK_32x32, 32, 32, 8, 11.7, 1.1},
+                                  {KUDNN_CFG_WAVEK_64x32, 64, 32, 6, 11.3, 1.1}, {KUDNN_CFG_WAVEK_32x64, 32, 64, 6, 11.8, 1.1},
+                                  {KUDNN_CFG_WAVEK_64x64, 64, 64, 8, 12.6, 1.25}, {KUDNN_CFG_WAVEK_64x64_W4, 64, 64, 4, 12.9, 1.1},
+                                  {KUDNN_CFG_WAVEK_64x128, 64, 128, 4, 15.5, 1.1}};
+    const bool f16w8 = weight8 && ct != KUDNN_DT_S8;          // two 128-byte pieces of an A row a k-tile
+    const int64_t bk = weight8 || ct == KUDNN_DT_S8 ? 128 : 64;
+    const int64_t KT = (K + bk - 1) / bk;
+    if ((bk == 64 && (M <= 16 || (M >= 256 && M % 128 == 0))) || K < 4 * bk) {
         return 0;
     }
-    const double hbm = static_cast<double>(N) * static_cast<double>(K) * 2.0 / 6.6e6;
+    const double mac = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K * batches);
+    const double mfma = mac * 2.0 / (ct == KUDNN_DT_S8 ? 1.4e9 : 0.8e9);
+    const double hbm = static_cast<double>(N) * static_cast<double>(K) * (bk == 128 ? 1.0 : 2.0) / 6.6e6;
     int best = 0;
     double bestUs = 0.0;
     for (const Tile &t : kTiles) {
-        if (kmajor && t.bn < 64) {
+        if ((kmajor && t.bn < 64) || (t.bm == 16 && (M > 16 || bk == 64))) {
             continue;
         }
+        const int64_t waves = f16w8 && t.bm == 64 && t.bn == 64 ? t.waves * 3 / 4 : t.waves;
+        const double kb = (t.bm * (f16w8 ? 2 : 1) + t.bn) / 8.0;  // KB of a k-tile: a wave's stage
         const int64_t tiles = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn) * batches;
-        const int64_t perCu = (tiles + 255) / 256, ktiles = (KT + t.waves - 1) / t.waves * t.waves;
-        const double copies = static_cast<double>(perCu * ktiles) * (t.bm + t.bn) / 8.0 * t.nsPerKB * 1e-3 *
-                              (perCu > t.fit ? 1.1 : 1.0);
-        const double us = 4.2 + (copies > hbm ? copies + 0.15 * hbm : hbm + 0.15 * copies);
+        const int64_t perCu = (tiles + 255) / 256, ktiles = (KT + waves - 1) / waves * waves;
+        const double copies = static_cast<double>(perCu * ktiles) * kb * t.nsPerKB * 1e-3 *
+                              (static_cast<double>(perCu * waves) * kb > 160.0 ? t.over : 1.0);
+        const double busy = copies > mfma ? copies : mfma;
+        const double us = 4.2 + (busy > hbm ? busy + 0.15 * hbm : hbm + 0.15 * copies);
         if (best == 0 || us < bestUs) {
             best = t.cfg;
             bestUs = us;

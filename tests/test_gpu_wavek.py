@@ -11,7 +11,7 @@ from test_gpu_layouts import T, run_gemm
 
 torch = pytest.importorskip("torch")
 
-TILES = {"30": "32x16_w8", "31": "32x32_w8", "32": "32x64_w6", "33": "64x32_w6", "34": "64x64_w8", "35": "64x64_w4",
+TILES = {"28": "16x16_w8", "29": "16x32_w8", "30": "32x16_w8", "31": "32x32_w8", "32": "32x64_w6", "33": "64x32_w6", "34": "64x64 ", "35": "64x64_2percu",
          "36": "64x128_w4"}
 WIDE = ("32", "34", "35", "36")  # the tiles that read a [K][N] weight in place
 
@@ -25,7 +25,7 @@ def gpu():
 
 # K: one chunk, one k-tile, a k-tile and a chunk, fewer k-tiles than waves, one each, one more; odd (packed)
 @pytest.mark.gpu
-@pytest.mark.parametrize("cfg", list(TILES))
+@pytest.mark.parametrize("cfg", list(TILES)[2:])
 @pytest.mark.parametrize("M,N,Kd", [(17, 16, 8), (32, 33, 64), (33, 130, 72), (64, 128, 320), (65, 264, 512), (70, 40, 584),
                                     (255, 7, 1000), (40, 72, 131)])
 @pytest.mark.parametrize("dt", [O.BF16, O.F16])
@@ -36,13 +36,48 @@ def test_tiles_exact(gpu, monkeypatch, cfg, M, N, Kd, dt):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("cfg", list(TILES))
+@pytest.mark.parametrize("cfg", list(TILES)[2:])
 @pytest.mark.parametrize("M,N,Kd", [(17, 8, 64), (64, 128, 448), (70, 200, 512), (130, 264, 64), (33, 72, 200), (33, 70, 128)])
 def test_kmajor_weight_exact(gpu, monkeypatch, cfg, M, N, Kd):
     # [K][N]: in place by the wide tiles when N is a multiple of 8 and K of 64, packed otherwise
     monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
     d, _ = run_gemm(T([M, Kd], O.BF16), T([Kd, N], O.BF16, "AB"), T([M, N], O.F32), None, seed=851, int_valued=True)
     assert ("kmajorB" in d) == (cfg in WIDE and N % 8 == 0 and Kd % 64 == 0), d
+
+
+# 8-bit weights: K of one chunk, one k-tile (128), a k-tile and a chunk, k-tiles for every wave and more; K = 200 is no
+# whole number of chunks, so the operands are packed
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", list(TILES))
+@pytest.mark.parametrize("M,N,Kd", [(1, 16, 16), (16, 33, 128), (17, 130, 144), (64, 128, 1040), (70, 40, 1168), (130, 264, 200)])
+@pytest.mark.parametrize("adt,bdt,cdt", [(O.F16, O.S8, O.F32), (O.F16, O.U8, O.F32), (O.S8, O.S8, O.S32), (O.U8, O.S8, O.S32)])
+def test_8bit_weights_exact(gpu, monkeypatch, cfg, M, N, Kd, adt, bdt, cdt):
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
+    bias = T([1, N], O.S32 if cdt == O.S32 else O.F32)
+    d, _ = run_gemm(T([M, Kd], adt), T([Kd, N], bdt, "BA"), T([M, N], cdt), bias, seed=855, int_valued=True)
+    assert TILES[cfg] in d and ("pack" in d) == (Kd % 16 != 0), d
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("adt,bdt,cdt", [(O.F16, O.S8, O.F16), (O.U8, O.S8, O.S32)])
+def test_8bit_unaligned_base(gpu, adt, bdt, cdt):
+    # operands that start off a 16-byte boundary are packed at run time, whatever the plan found in their strides
+    M, N, Kd = 20, 96, 1024
+    a, b = Case([M, Kd], adt, seed=856, lo=-1.0 if adt == O.F16 else 0, hi=1.0 if adt == O.F16 else 255), \
+        Case([Kd, N], bdt, "BA", seed=857, lo=-128, hi=127)
+    c = Case([M, N], cdt, zero=True)
+    plan = K.Gemm(a.desc, b.desc, c.desc)
+    assert "wavek" in plan.describe() and "pack" not in plan.describe(), plan.describe()
+    ref = c.clone_empty()
+    O.gemm(a.t, b.t, ref)
+    for off_a, off_b in ((0, 0), (1, 0), (0, 1), (1, 1)):
+        da, db = a.device(), b.device()
+        pa = torch.zeros(da.numel() + 8, dtype=da.dtype, device="cuda")[off_a:off_a + da.numel()].copy_(da)
+        pb = torch.zeros(db.numel() + 16, dtype=db.dtype, device="cuda")[off_b:off_b + db.numel()].copy_(db)
+        dc = zeros_device(c)
+        plan.run(pa, pb, dc)
+        torch.cuda.synchronize()
+        compare(from_device(dc, cdt), ref.buf, cdt, f"{off_a} {off_b} {plan.describe()}")
 
 
 @pytest.mark.gpu
@@ -111,3 +146,15 @@ def test_planner_rule():
     assert "pack" not in plan(100, 1000, 4096) and "packA packB" in plan(100, 1001, 4096)
     assert plan(16, 4096, 4096).startswith("skinny") and "wavek" not in plan(256, 4096, 4096)
     assert "wavek" not in plan(255, 4096, 14336) and "wavek" not in plan(40, 128, 4096)
+    # 8-bit weights: from M = 1, K of at least 4 k-tiles of 128 (the last may be partial) in whole 16-byte chunks
+
+    def plan8(M, Kd, N, adt, bdt, cdt):
+        return K.Gemm(K.desc([M, Kd], adt), K.desc([Kd, N], bdt, "BA"), K.desc([M, N], cdt)).describe()
+    assert plan8(4, 4096, 4096, K.F16, K.S8, K.F16).startswith("mfma_f16_wavek_16x16")
+    assert "pack" not in plan8(64, 1040, 4096, K.F16, K.U8, K.F16)
+    assert "packB" in plan8(4, 1000, 4096, K.F16, K.S8, K.F16) and "packB" in plan8(4, 384, 4096, K.F16, K.S8, K.F16)
+    assert plan8(64, 4096, 4096, K.S8, K.S8, K.S32).startswith("mfma_s8_wavek")
+    assert "pack" not in plan8(64, 4096, 4096, K.U8, K.S8, K.S32)
+    assert "wavek" not in plan8(64, 4096, 4096, K.S8, K.U8, K.S32) and "wavek" not in plan8(1024, 4096, 4096, K.S8, K.S8, K.S32)
+    assert "wavek" in plan8(1024, 4096, 4096, K.U8, K.S8, K.S32) and "wavek" not in plan8(2048, 4096, 11008, K.U8, K.S8, K.S32)
+    assert "wavek" in plan(400, 4096, 4096) and "wavek" not in plan(512, 4096, 4096) and "wavek" not in plan(1000, 4096, 11008)
