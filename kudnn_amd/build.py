@@ -26,7 +26,7 @@ BUILD = PKG / "_build"
 INCLUDE = ROOT / "include"
 
 ARCH = os.environ.get("KUDNN_OFFLOAD_ARCH", "gfx950")
-HIP_SOURCES = ["gemm_mfma.hip", "gemm_pingpong.hip", "gemm_kslice.hip", "gemm_wavek.hip", "skinny_bf16.hip", "pack.hip", "capi.cpp"]
+HIP_SOURCES = ["gemm_mfma.hip", "gemm_pingpong.hip", "gemm_kslice.hip", "gemm_wavek.hip", "gemm_wavek8.hip", "skinny_bf16.hip", "pack.hip", "capi.cpp"]
 HIP_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",
@@ -85,7 +85,7 @@ def build_hip(verbose: bool = False) -> Path:
         objs.append(obj)
         extra = [f'-DKUDNN_PINGPONG_DIGEST="{pingpong_digest()}"'] if src == "gemm_pingpong.hip" else []
         jobs.append([hipcc, *HIP_FLAGS, *extra, "-c", str(CSRC / src), "-o", str(obj)])
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(4, len(jobs))) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(jobs))) as ex:
         list(ex.map(lambda c: _run(c, verbose), jobs))
     out = LIB / "libkudnn_hip.so"
     tmp = LIB / "libkudnn_hip.so.tmp"

@@ -549,17 +549,26 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
                           core.B.bs[2] % 8 == 0 && core.K % 64 == 0 && core.N % 8 == 0 &&
                           !std::getenv("KUDNN_HIP_PACK_KMAJOR");
 
-    // Whether the wave-K kernel can read both operands in place: contiguous along K in whole 16-byte chunks (it masks the
-    // K tail itself), of the compute type, a u8 A of an integer product, or an 8-bit weight of an f16 product.
+    // What the wave-K kernel can read in place. It masks the K tail itself; rows that lie contiguous along K in whole
+    // 16-byte chunks go through the LDS DMA (`chunked`), rows of any other alignment through registers (`byRow`); the
+    // types are the compute type's own, a u8 A of an integer product, or an 8-bit weight of an f16 product. A 16-bit
+    // weight stored [K][N] takes whole chunks of columns (kmajorWk). Weights under 4 MB that the other kernels would pack
+    // for their K keep those packs: two short launches, and no gain was measured there.
     const auto chunked = [&](const OperandSpec &o) {
         const int64_t c = 16 / DtSize(o.dt);
         return o.s_k == 1 && core.K % c == 0 && o.s_r % c == 0 && o.bs[0] % c == 0 && o.bs[1] % c == 0 && o.bs[2] % c == 0;
     };
-    const bool inPlaceA = chunked(core.A) && (core.A.dt == core.computeDt ||
-                                              (core.computeDt == KUDNN_DT_S8 && core.A.dt == KUDNN_DT_U8));
     const bool w8 = core.computeDt == KUDNN_DT_F16 && (core.B.dt == KUDNN_DT_S8 || core.B.dt == KUDNN_DT_U8);
-    const bool inPlaceAB = inPlaceA && chunked(core.B) && (core.B.dt == core.computeDt || w8);
-    const bool weight8 = w8 && inPlaceAB;
+    const bool typesWk = (core.A.dt == core.computeDt || (core.computeDt == KUDNN_DT_S8 && core.A.dt == KUDNN_DT_U8)) &&
+                         (core.B.dt == core.computeDt || w8);
+    const bool largeB = core.N * core.K * DtSize(core.B.dt) >= (int64_t(4) << 20);
+    const bool chunkedAB = typesWk && chunked(core.A) && chunked(core.B);
+    const bool byRow = typesWk && !chunkedAB && core.A.s_k == 1 && core.B.s_k == 1 && core.K >= 16 && largeB;
+    const bool kmajorWk = kmajor16 || (largeB && lowp16 && core.B.dt == core.computeDt && core.B.s_r == 1 &&
+                                       core.B.s_k >= core.N && core.B.s_k % 8 == 0 && core.B.bs[0] % 8 == 0 &&
+                                       core.B.bs[1] % 8 == 0 && core.B.bs[2] % 8 == 0 && core.N % 8 == 0 &&
+                                       !std::getenv("KUDNN_HIP_PACK_KMAJOR"));
+    const bool weight8 = w8 && (chunkedAB || byRow);
 
     // engine and tile configuration
     const int64_t batches = core.Batches();
@@ -621,11 +630,14 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         } else if (core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256) {
             other = S >= 2 ? 9.0 + 1.2 * kt / S + S * mn * 8.0 / 3.6e6 : 5.0 + 1.15 * kt * static_cast<double>((t256 + 255) / 256);
         }
-        other += weight8 ? 3.0 + nk * 0.75e-6 : (s8 && core.A.dt == KUDNN_DT_U8 ? 14.0 + nk * 0.47e-6 : 0.0);
+        const double bytesAB = static_cast<double>(core.M * core.K * DtSize(core.A.dt) + core.N * core.K * DtSize(core.B.dt));
+        const bool packs = byRow || core.K % bk != 0;  // the other kernels pack both operands to whole k-tiles
+        other += weight8 ? 3.0 + nk * 0.75e-6 : (s8 && core.A.dt == KUDNN_DT_U8 ? 14.0 + nk * 0.47e-6
+                                                                                : (packs ? 5.0 + bytesAB * 2.0 / 4.2e6 : 0.0));
         // an integer product with a u8 weight needs row sums of A, and an 8-bit weight of an f16 product that cannot be
         // read in place is packed to f16: both stay with the other kernels
-        if (core.B.dt != KUDNN_DT_U8 || weight8) {
-            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, core.computeDt, weight8, kmajor16, other)) {
+        if ((core.B.dt != KUDNN_DT_U8 || weight8) && (core.M > 16 || !lowp16 || weight8 || byRow)) {
+            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, core.computeDt, weight8, kmajorWk, byRow, other)) {
                 core.engine = ENGINE_MFMA_BF16;
                 core.cfg = wk;
             }
@@ -649,6 +661,31 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         if (t64 < KUDNN_SPLIT_MAX_TILES && tks >= 128 && (core.kp <= 4096 || core.M <= 16)) {
             core.cfg = KUDNN_CFG_F32_KSLICE_16x32;
         }
+        // Both operands contiguous along K: the wave-K tiles where their estimate beats the choice above. The k-slice
+        // kernel's 4-wave form (K not whole 256-element blocks) took 3 us + 5.2 ns per k and round of 256 tiles, its
+        // whole-line form 2.5 + 3.2 ns; a 64 x 64 grid split over workgroups about 20 us, unsplit 0.38 TFLOP/s a CU in
+        // one round and 0.45 in more, 128 x 128 tiles 0.5; K off the 32-deep k-tile adds the packs.
+        if ((chunkedAB || byRow) && t64 >= 16) {
+            const double bytesAB = static_cast<double>((core.M + core.N) * core.K) * 4.0;
+            const double k = static_cast<double>(core.kp);
+            double other = 0.0;
+            if (core.cfg == KUDNN_CFG_F32_KSLICE_16x32) {
+                const double rounds = static_cast<double>((tks + 255) / 256);
+                other = kudnn_kslice_whole_line(core.kp) ? 2.5 + 3.2e-3 * k * rounds : 3.0 + 5.2e-3 * k * rounds;
+            } else if (core.cfg == KUDNN_CFG_F32_64x64) {
+                other = 4.0 + static_cast<double>((t64 + 255) / 256) * k * (64 * 64 * 2e-6) / (t64 <= 256 ? 0.38 : 0.45);
+                if (t64 < KUDNN_SPLIT_MAX_TILES) {
+                    other = std::max(other / 2, 20.0);
+                }
+            } else {
+                other = 4.0 + static_cast<double>((t128 + 255) / 256) * k * (128 * 128 * 2e-6) / 0.5;
+            }
+            other += core.K % bk != 0 ? 5.0 + bytesAB * 2.0 / 4.2e6 : 0.0;
+            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, core.computeDt, false, false, byRow, other)) {
+                core.engine = ENGINE_MFMA_BF16;
+                core.cfg = wk;
+            }
+        }
     }
     if (const char *force = std::getenv("KUDNN_HIP_FORCE_CFG")) {
         int f = std::atoi(force);
@@ -658,34 +695,39 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         bool okBf16 = core.computeDt != KUDNN_DT_F32 &&
                       (((f == KUDNN_CFG_BF16_256x256 || f == KUDNN_CFG_BF16_256x128 || f == KUDNN_CFG_BF16_128x128 ||
                          f == KUDNN_CFG_BF16_PINGPONG_256x256) && mfmaOk) ||
-                       (kudnn_is_wavek(f) && (lowp16 || core.B.dt == KUDNN_DT_S8)) ||
+                       (kudnn_is_wavek(f) && (lowp16 || core.B.dt == KUDNN_DT_S8) && (core.M > 16 || weight8 || byRow || !lowp16)) ||
                        (f == KUDNN_CFG_SKINNY_BF16 && core.M >= 2 && core.M <= 16 && lowp16) ||
                        (f == KUDNN_CFG_GEMV_MULTI_BF16 && core.M >= 2 && core.M <= 8 && lowp16) ||
                        (f == KUDNN_CFG_GEMV_KSPLIT_BF16 && core.M >= 2 && core.M <= 16 && lowp16));
         bool okF32 = core.computeDt == KUDNN_DT_F32 &&
-                     (f == KUDNN_CFG_F32_128x128 || f == KUDNN_CFG_F32_64x64 || f == KUDNN_CFG_F32_KSLICE_16x32);
+                     (f == KUDNN_CFG_F32_128x128 || f == KUDNN_CFG_F32_64x64 || f == KUDNN_CFG_F32_KSLICE_16x32 ||
+                      (kudnn_is_wavek(f) && (chunkedAB || byRow)));
         if (okBf16 || okF32) {
             core.cfg = f;
             const bool skinny = f == KUDNN_CFG_SKINNY_BF16 || f == KUDNN_CFG_GEMV_MULTI_BF16 || f == KUDNN_CFG_GEMV_KSPLIT_BF16;
-            core.engine = skinny ? ENGINE_SKINNY_BF16 : (okF32 ? ENGINE_MFMA_F32 : ENGINE_MFMA_BF16);
+            core.engine = skinny ? ENGINE_SKINNY_BF16 : (okF32 && !kudnn_is_wavek(f) ? ENGINE_MFMA_F32 : ENGINE_MFMA_BF16);
         }
     }
     // A K-major weight (B stored [K][N], N contiguous: C5's W{1,K,N} ABC) is read in place by the ping-pong kernel,
     // through transposing LDS reads, instead of being packed on every run; it needs 64-deep k-tiles, N a multiple of
     // 8 (whole 16-byte column chunks; an edge tile's columns past N are computed and never stored), 16-byte aligned
     // k-rows and batches, and 32-bit offsets. The wave-K tiles of 64 and 128 columns do the same with 64-bit addresses.
-    const bool wavek = core.engine == ENGINE_MFMA_BF16 && kudnn_is_wavek(core.cfg);
+    const bool wavek = kudnn_is_wavek(core.cfg);
     const bool wide = core.cfg == KUDNN_CFG_WAVEK_32x64 || core.cfg == KUDNN_CFG_WAVEK_64x64 ||
                       core.cfg == KUDNN_CFG_WAVEK_64x64_W4 || core.cfg == KUDNN_CFG_WAVEK_64x128;
-    if (kmajor16 && ((wavek && wide) ||
-                     (core.engine == ENGINE_MFMA_BF16 && core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256 &&
-                      core.K * core.B.s_k * 2 < (int64_t(1) << 31) &&
-                      core.M * std::max<int64_t>(core.A.s_r, core.kp) * 2 < (int64_t(1) << 31)))) {
+    if ((wavek && kmajorWk && wide) ||
+        (kmajor16 && core.engine == ENGINE_MFMA_BF16 && core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256 &&
+         core.K * core.B.s_k * 2 < (int64_t(1) << 31) &&
+         core.M * std::max<int64_t>(core.A.s_r, core.kp) * 2 < (int64_t(1) << 31))) {
         core.B.kmajor = true;
         core.B.staticPack = false;
     }
-    if (wavek && !core.B.kmajor && inPlaceAB) {
-        core.A.staticPack = core.B.staticPack = false;
+    if (wavek) {
+        if (chunkedAB || byRow) {
+            core.A.staticPack = core.B.staticPack = false;
+        } else if (core.B.kmajor && core.A.dt == core.computeDt) {
+            core.A.staticPack = !chunked(core.A);
+        }
     }
     // The same for an fp32 weight stored [K][N] (the reference's Matmul mode passes W in ABCDE,
     // matmul_gtest.cpp:248-257), read in place by the 4-wave fp32 kernels (128 x 128 and 64 x 64) and by the k-slice
@@ -732,8 +774,14 @@ const char *CfgName(int cfg)
 
 std::string DescribeCore(const GemmCore &c)
 {
-    // the 16- and 8-bit configurations carry the bf16 names; name the operand type actually computed
+    // the 16- and 8-bit configurations carry the bf16 names; name the operand type actually computed. The wave-K tiles
+    // are the decode kernel of 16-bit operands that the others would pack, and another form of the f32 k-slice kernel.
     std::string cfg = CfgName(c.cfg);
+    if (kudnn_is_wavek(c.cfg) && c.computeDt == KUDNN_DT_F32) {
+        cfg.replace(0, std::strlen("mfma_bf16_wavek"), "mfma_f32_kslice");
+    } else if (kudnn_is_wavek(c.cfg) && c.computeDt != KUDNN_DT_S8 && c.M <= 16 && DtSize(c.B.dt) == 2) {
+        cfg.replace(0, std::strlen("mfma"), "skinny");
+    }
     const char *ct = c.computeDt == KUDNN_DT_F16 ? "f16" : (c.computeDt == KUDNN_DT_S8 ? "s8" : nullptr);
     const size_t at = cfg.find("bf16");
     if (ct != nullptr && at != std::string::npos) {
@@ -957,7 +1005,7 @@ int LaunchCore(const GemmCore &core, const EpiExtras &x, const void *a, const vo
     op.N = core.N;
     // MFMA kernels run whole k-tiles: when K is not a multiple of the tile both operands were packed with
     // zero padding up to kp (and kp == K otherwise). The skinny and wave-K kernels mask their own K tail.
-    const bool wavek = core.engine == ENGINE_MFMA_BF16 && kudnn_is_wavek(core.cfg);
+    const bool wavek = kudnn_is_wavek(core.cfg);
     op.K = core.engine == ENGINE_SKINNY_BF16 || wavek ? core.K : core.kp;
     auto setupOperand = [&](const OperandSpec &o, const void *ptr, bool pack, void *dst, const void *&outPtr,
                             int64_t &ld, int64_t outBs[3]) -> int {
@@ -1158,6 +1206,7 @@ int LaunchCore(const GemmCore &core, const EpiExtras &x, const void *a, const vo
             // the weight's type as the kernel finds it; u8 under s8 stands for a u8 A
             const int bt = core.computeDt == KUDNN_DT_S8 ? core.A.dt : (packB ? core.computeDt : core.B.dt);
             op.a_u8 = aU8 && !packA ? 1 : 0;
+            op.k_padded = packA && (packB || op.b_kmajor) ? 1 : 0;
             lrc = kudnn_launch_gemm_wavek(op, ep, batches, core.computeDt, bt, core.cfg, stream);
         } else if (core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256 && kudnn_pingpong_eligible(op, core.computeDt)) {
             lrc = kudnn_launch_gemm_pingpong(op, ep, batches, core.computeDt, tailWs, slicesOk, stream);

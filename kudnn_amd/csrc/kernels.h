@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "plan_types.h"
 
 // Tile configurations of the dispatcher (values are stable: they appear in plan descriptions).
@@ -105,19 +107,28 @@ inline int kudnn_tail_slice_rule(int64_t M, int64_t N, int64_t KT, int64_t batch
     return S >= 2 ? static_cast<int>(S) : 0;
 }
 
-// Tiles whose K is dealt to the workgroup's waves (gemm_wavek.hip): 16-byte aligned rows and bases; op.K is the true K
-// (whole 16-byte chunks, or rows packed with zeros up to whole chunks); b_kmajor (16-bit) with N and ldb multiples of 8
-// and the tiles of 64 or 128 columns. `bt` is the weight's stored type: ct, s8 or u8 under f16, and u8 under s8 for a u8
+// The wave-K tiles that can take rows of any alignment through registers (the wider ones have none to spare).
+constexpr bool kudnn_wavek_reg_tile(int bm, int bn, int waves)
+{
+    return bn >= bm / 2 && bm * bn <= 64 * 64 && (bm * bn < 64 * 64 || waves <= 4) && (bm != 32 || bn != 16);
+}
+
+// Tiles whose K is dealt to the workgroup's waves (gemm_wavek.hip). op.K is the true K; k_padded says that packed rows
+// hold zeros up to a whole 16-byte chunk. Operands that are not whole chunks (rows, K, bases) take the register form.
+// b_kmajor (16-bit): whole chunks of columns, tiles of 32 columns or more. `bt` is the weight's stored type: ct, s8 or u8 under f16, and u8 under s8 for a u8
 // A beside an s8 weight (the term of the -128 shift is added here; op.a_u8 says whether A still has to be shifted). No
 // workspace.
 int kudnn_launch_gemm_wavek(const GemmOperands &op, const EpiParams &ep, int64_t batches, int ct, int bt, int cfg,
                             hipStream_t stream);
+// Its 8-bit and f32 instances (a translation unit of their own); `reg`: the register form.
+int kudnn_launch_gemm_wavek8(const GemmOperands &op, const EpiParams &ep, int64_t batches, int ct, int bt, int cfg, bool reg,
+                             hipStream_t stream);
 
 // The wave-K tile for a product (0: the kernel the other rules chose). The estimate is what the measurements of 7 tiles
 // over M = 17..1030 and N, K = 2048..14336 (weights rotated past the Infinity Cache) fit: 4.2 us a call, plus the largest
 // of the weight's stream from HBM at 6.6 TB/s, the busiest CU's copies, nsPerKB per KB of A and B (`over` times that when
-// more tiles come to a CU than fit beside one another), and the products at 0.8 PFLOP/s (8-bit: 1.4), plus a part of the
-// stream. Over 26 drawn bf16 shapes the choice was within 7 % of the best tile but for 3 (19 %). otherUs is the same kind
+// more tiles come to a CU than fit beside one another), and the products at 0.8 PFLOP/s (8-bit 1.4; f32 by the tile's rate on the
+// busiest CU), plus a part of the stream. Over 26 drawn bf16 shapes the choice was within 7 % of the best tile but for 3 (19 %). otherUs is the same kind
 // of estimate for the other rules' kernel (BuildCore). Measured, against the other kernel: bf16 64 x 4096 x 4096 10 us (31),
 // 64 x 11008 x 4096 22 (48), 192 x 4096 x 11008 45 (48), 400 x 4096 x 4096 27 (45); f16 x s8 4 x 4096 x 4096 6.1 (21.5),
 // 128 x 4096 x 4096 12 (55); u8 x s8 64 x 4096 x 4096 7.5 (47), 1024 x 4096 x 4096 40 (51). The others stay where a weight
@@ -126,40 +137,46 @@ int kudnn_launch_gemm_wavek(const GemmOperands &op, const EpiParams &ep, int64_t
 // 256 rows or more in whole 128-row tiles keep the plans that the dispatch sweep fixed for them. Less than 4 whole
 // k-tiles leave most waves without one.
 inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, int ct, bool weight8, bool kmajor,
-                            double otherUs)
+                            bool byRow, double otherUs)
 {
     struct Tile {
         int cfg, bm, bn, waves;
-        double nsPerKB, over;
+        double nsPerKB, over, f32Rate;  // f32Rate: f32 TFLOP/s of a CU
     };
-    static const Tile kTiles[] = {{KUDNN_CFG_WAVEK_16x16, 16, 16, 8, 11.5, 1.1}, {KUDNN_CFG_WAVEK_16x32, 16, 32, 8, 11.6, 1.1},
-                                  {KUDNN_CFG_WAVEK_32x16, 32, 16, 8, 11.5, 1.1}, {KUDNN_CFG_WAVEK_32x32, 32, 32, 8, 11.7, 1.1},
-                                  {KUDNN_CFG_WAVEK_64x32, 64, 32, 6, 11.3, 1.1}, {KUDNN_CFG_WAVEK_32x64, 32, 64, 6, 11.8, 1.1},
-                                  {KUDNN_CFG_WAVEK_64x64, 64, 64, 8, 12.6, 1.25}, {KUDNN_CFG_WAVEK_64x64_W4, 64, 64, 4, 12.9, 1.1},
-                                  {KUDNN_CFG_WAVEK_64x128, 64, 128, 4, 15.5, 1.1}};
+    static const Tile kTiles[] = {{KUDNN_CFG_WAVEK_16x16, 16, 16, 8, 11.5, 1.1, 0.25}, {KUDNN_CFG_WAVEK_16x32, 16, 32, 8, 11.6, 1.1, 0.28},
+                                  {KUDNN_CFG_WAVEK_32x16, 32, 16, 8, 11.5, 1.1, 0.28}, {KUDNN_CFG_WAVEK_32x32, 32, 32, 8, 11.7, 1.1, 0.32},
+                                  {KUDNN_CFG_WAVEK_64x32, 64, 32, 6, 11.3, 1.1, 0.32}, {KUDNN_CFG_WAVEK_32x64, 32, 64, 6, 11.8, 1.1, 0.32},
+                                  {KUDNN_CFG_WAVEK_64x64, 64, 64, 8, 12.6, 1.25, 0.34}, {KUDNN_CFG_WAVEK_64x64_W4, 64, 64, 4, 12.9, 1.1, 0.44},
+                                  {KUDNN_CFG_WAVEK_64x128, 64, 128, 4, 15.5, 1.1, 0.48}};
     const bool f16w8 = weight8 && ct != KUDNN_DT_S8;          // two 128-byte pieces of an A row a k-tile
-    const int64_t bk = weight8 || ct == KUDNN_DT_S8 ? 128 : 64;
+    const bool f32 = ct == KUDNN_DT_F32;
+    const int64_t bk = f32 ? 32 : (weight8 || ct == KUDNN_DT_S8 ? 128 : 64);
     const int64_t KT = (K + bk - 1) / bk;
-    if ((bk == 64 && (M <= 16 || (M >= 256 && M % 128 == 0))) || K < 4 * bk) {
+    if ((bk == 64 && M >= 256 && M % 256 == 0 && K % 64 == 0) || K < 4 * bk) {
         return 0;
     }
     const double mac = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K * batches);
-    const double mfma = mac * 2.0 / (ct == KUDNN_DT_S8 ? 1.4e9 : 0.8e9);
-    const double hbm = static_cast<double>(N) * static_cast<double>(K) * (bk == 128 ? 1.0 : 2.0) / 6.6e6;
+    const double stream = static_cast<double>(N) * static_cast<double>(K) * 128.0 / static_cast<double>(bk) / 6.6e6;
     int best = 0;
     double bestUs = 0.0;
     for (const Tile &t : kTiles) {
-        if ((kmajor && t.bn < 64) || (t.bm == 16 && (M > 16 || bk == 64))) {
+        if ((kmajor && t.bn < 64) || (t.bm == 16 && (M > 16 || (bk == 64 && !byRow))) ||
+            (byRow && !kudnn_wavek_reg_tile(t.bm, t.bn, t.waves))) {
             continue;
         }
         const int64_t waves = f16w8 && t.bm == 64 && t.bn == 64 ? t.waves * 3 / 4 : t.waves;
         const double kb = (t.bm * (f16w8 ? 2 : 1) + t.bn) / 8.0;  // KB of a k-tile: a wave's stage
         const int64_t tiles = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn) * batches;
         const int64_t perCu = (tiles + 255) / 256, ktiles = (KT + waves - 1) / waves * waves;
-        const double copies = static_cast<double>(perCu * ktiles) * kb * t.nsPerKB * 1e-3 *
+        const double copies = static_cast<double>(perCu * ktiles) * kb * t.nsPerKB * (byRow ? 1.15e-3 : (kmajor ? 1.08e-3 : 1e-3)) *
                               (static_cast<double>(perCu * waves) * kb > 160.0 ? t.over : 1.0);
+        const double mfma = f32 ? static_cast<double>(perCu * t.bm * t.bn) * 2e-6 * static_cast<double>(ktiles * bk) / t.f32Rate
+                                : mac * 2.0 / (ct == KUDNN_DT_S8 ? 1.4e9 : 0.8e9);
+        // a part of the CUs streams a part of HBM's rate: in proportion for k-rows, less so for rows
+        const double part = tiles < 256 ? 256.0 / static_cast<double>(tiles) : 1.0;
+        const double hbm = stream * (kmajor ? part : std::sqrt(part));
         const double busy = copies > mfma ? copies : mfma;
-        const double us = 4.2 + (busy > hbm ? busy + 0.15 * hbm : hbm + 0.15 * copies);
+        const double us = 4.2 + (busy > hbm ? busy + 0.15 * stream : hbm + 0.15 * copies);
         if (best == 0 || us < bestUs) {
             best = t.cfg;
             bestUs = us;

@@ -52,6 +52,7 @@ struct GemmOperands {
     int64_t lda, ldb;
     int64_t a_bs[3], b_bs[3];  // batch strides (elements), same batch dims as EpiParams::bdim
     int a_u8;      // 1: A is u8 as stored, to be shifted by -128 in registers (the wave-K kernel's integer products)
+    int k_padded;  // 1: the rows of A (and of a B stored [N][K]) hold zeros from K up to a whole 16-byte chunk (packed)
     int b_kmajor;  // 1: B is stored [K][N] (N contiguous, row pitch ldb along k): the 16-bit ping-pong kernel and the
                    // 4-wave fp32 kernels read it
 };

@@ -14,6 +14,7 @@ torch = pytest.importorskip("torch")
 TILES = {"28": "16x16_w8", "29": "16x32_w8", "30": "32x16_w8", "31": "32x32_w8", "32": "32x64_w6", "33": "64x32_w6", "34": "64x64 ", "35": "64x64_2percu",
          "36": "64x128_w4"}
 WIDE = ("32", "34", "35", "36")  # the tiles that read a [K][N] weight in place
+ROWS = ("28", "29", "31", "32", "33", "35")  # the tiles that read unaligned rows (from 4 MB of weight on)
 
 
 @pytest.fixture
@@ -80,6 +81,53 @@ def test_8bit_unaligned_base(gpu, adt, bdt, cdt):
         compare(from_device(dc, cdt), ref.buf, cdt, f"{off_a} {off_b} {plan.describe()}")
 
 
+# rows of any alignment, read through registers: K ends 1, 3, 4, 7 elements into a 16-byte chunk (f32: 1, 3)
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", ROWS)
+@pytest.mark.parametrize("M,N,Kd", [(5, 4200, 1009), (33, 8500, 523), (70, 1041, 4103), (16, 4099, 1028)])
+@pytest.mark.parametrize("adt,bdt,cdt", [(O.BF16, O.BF16, O.F32), (O.F16, O.F16, O.F32), (O.F16, O.S8, O.F32), (O.F16, O.U8, O.F32),
+                                         (O.S8, O.S8, O.S32), (O.U8, O.S8, O.S32), (O.F32, O.F32, O.F32)])
+def test_unaligned_rows_exact(gpu, monkeypatch, cfg, M, N, Kd, adt, bdt, cdt):
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
+    if adt == O.F16 and bdt != O.F16 and Kd > 4000:
+        Kd = 4099  # 16 x 255 x 4099 stays below 2^24
+    d, _ = run_gemm(T([M, Kd], adt), T([Kd, N], bdt, "BA"), T([M, N], cdt), None, seed=858, int_valued=True)
+    assert TILES[cfg].split("_")[0] in d and "pack" not in d, d
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", list(TILES))
+@pytest.mark.parametrize("M,N,Kd", [(17, 16, 4), (32, 33, 32), (33, 130, 72), (64, 128, 320), (255, 7, 1000), (70, 264, 256)])
+def test_f32_tiles_exact(gpu, monkeypatch, cfg, M, N, Kd):
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
+    d, _ = run_gemm(T([M, Kd], O.F32), T([Kd, N], O.F32, "BA"), T([M, N], O.F32), T([1, N], O.F32), seed=859, int_valued=True)
+    assert d.startswith("mfma_f32_kslice_" + TILES[cfg].strip()) and "pack" not in d, d
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", WIDE)
+@pytest.mark.parametrize("M,N,Kd", [(33, 2104, 1009), (64, 4200, 520)])
+def test_kmajor_weight_ragged_k_exact(gpu, monkeypatch, cfg, M, N, Kd):
+    # [K][N] with K off the k-tile, in place from 4 MB on; the source's rows are packed unless they are whole chunks
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
+    d, _ = run_gemm(T([M, Kd], O.BF16), T([Kd, N], O.BF16, "AB"), T([M, N], O.F32), None, seed=857, int_valued=True)
+    assert "kmajorB" in d and ("packA" in d) == (Kd % 8 != 0) and "packB" not in d, d
+
+
+@pytest.mark.gpu
+def test_f32_planner_against_float64(gpu):
+    # the planner's own choice for fp32 rows of any alignment: the error against 64 bits is that of f32 sums
+    for M, N, Kd in ((240, 1400, 1298), (100, 640, 3140), (33, 4000, 3002)):
+        x, w = torch.randn(M, Kd, device="cuda"), torch.randn(N, Kd, device="cuda")
+        y = torch.empty(M, N, device="cuda")
+        plan = K.Gemm(K.desc([M, Kd], K.F32), K.desc([Kd, N], K.F32, "BA"), K.desc([M, N], K.F32))
+        plan.run(x, w, y)
+        torch.cuda.synchronize()
+        ref = x.double() @ w.double().t()
+        # K products rounded and added in f32: a random walk of K roundings of 2^-24 each, times 4
+        assert float((y.double() - ref).norm() / ref.norm()) < 4 * 2.0 ** -24 * Kd ** 0.5, plan.describe()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("cfg", ["30", "35"])
 def test_batches_and_pitches_exact(gpu, monkeypatch, cfg):
@@ -142,9 +190,12 @@ def test_planner_rule():
     assert plan(17, 4096, 4096).startswith("mfma_bf16_wavek_32x16")
     assert plan(64, 4096, 4096, dt=K.F16).startswith("mfma_f16_wavek_32x32")
     assert plan(64, 4096, 11008).startswith("mfma_bf16_wavek_64x64")
-    assert "kmajorB" in plan(64, 4096, 4096, "AB") and "packA packB" in plan(64, 1000, 4096, "AB")
-    assert "pack" not in plan(100, 1000, 4096) and "packA packB" in plan(100, 1001, 4096)
+    assert "kmajorB" in plan(64, 4096, 4096, "AB") and "kmajorB" in plan(64, 1000, 4096, "AB")
+    assert "packA packB" in plan(64, 1000, 1024, "AB")
+    assert "pack" not in plan(100, 1000, 4096) and "pack" not in plan(100, 1001, 4096)
+    assert "packA packB" in plan(100, 1001, 1024)  # under 4 MB of weight
     assert plan(16, 4096, 4096).startswith("skinny") and "wavek" not in plan(256, 4096, 4096)
+    assert "wavek" not in plan(16, 4096, 4096) and plan(16, 4097, 4096).startswith("skinny_bf16_wavek_16x")
     assert "wavek" not in plan(255, 4096, 14336) and "wavek" not in plan(40, 128, 4096)
     # 8-bit weights: from M = 1, K of at least 4 k-tiles of 128 (the last may be partial) in whole 16-byte chunks
 
@@ -152,9 +203,14 @@ def test_planner_rule():
         return K.Gemm(K.desc([M, Kd], adt), K.desc([Kd, N], bdt, "BA"), K.desc([M, N], cdt)).describe()
     assert plan8(4, 4096, 4096, K.F16, K.S8, K.F16).startswith("mfma_f16_wavek_16x16")
     assert "pack" not in plan8(64, 1040, 4096, K.F16, K.U8, K.F16)
-    assert "packB" in plan8(4, 1000, 4096, K.F16, K.S8, K.F16) and "packB" in plan8(4, 384, 4096, K.F16, K.S8, K.F16)
+    assert "pack" not in plan8(4, 1001, 8192, K.F16, K.S8, K.F16) and "packB" in plan8(4, 1001, 2048, K.F16, K.S8, K.F16)
+    assert "packB" in plan8(4, 384, 4096, K.F16, K.S8, K.F16)
     assert plan8(64, 4096, 4096, K.S8, K.S8, K.S32).startswith("mfma_s8_wavek")
     assert "pack" not in plan8(64, 4096, 4096, K.U8, K.S8, K.S32)
     assert "wavek" not in plan8(64, 4096, 4096, K.S8, K.U8, K.S32) and "wavek" not in plan8(1024, 4096, 4096, K.S8, K.S8, K.S32)
     assert "wavek" in plan8(1024, 4096, 4096, K.U8, K.S8, K.S32) and "wavek" not in plan8(2048, 4096, 11008, K.U8, K.S8, K.S32)
     assert "wavek" in plan(400, 4096, 4096) and "wavek" not in plan(512, 4096, 4096) and "wavek" not in plan(1000, 4096, 11008)
+    def plan32(M, Kd, N):
+        return K.Gemm(K.desc([M, Kd], K.F32), K.desc([Kd, N], K.F32, "BA"), K.desc([M, N], K.F32)).describe()
+    assert plan32(107, 2176, 1984).startswith("mfma_f32_kslice_32x") and "pack" not in plan32(240, 1298, 1400)
+    assert plan32(128, 1024, 1024).startswith("mfma_f32_kslice_16x32") and plan32(2048, 4096, 4096).startswith("mfma_f32_128x128")
