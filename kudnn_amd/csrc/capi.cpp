@@ -553,7 +553,7 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
     // 16-byte chunks go through the LDS DMA (`chunked`), rows of any other alignment through registers (`byRow`); the
     // types are the compute type's own, a u8 A of an integer product, or an 8-bit weight of an f16 product. A 16-bit
     // weight stored [K][N] takes whole chunks of columns (kmajorWk). Weights under 4 MB that the other kernels would pack
-    // for their K keep those packs: two short launches, and no gain was measured there.
+    // for their K keep those packs: two short launches, and no gain was measured there (batches of products apart).
     const auto chunked = [&](const OperandSpec &o) {
         const int64_t c = 16 / DtSize(o.dt);
         return o.s_k == 1 && core.K % c == 0 && o.s_r % c == 0 && o.bs[0] % c == 0 && o.bs[1] % c == 0 && o.bs[2] % c == 0;
@@ -564,7 +564,7 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
     const bool largeB = core.N * core.K * DtSize(core.B.dt) >= (int64_t(4) << 20);
     const bool chunkedAB = typesWk && chunked(core.A) && chunked(core.B);
     const bool byRow = typesWk && !chunkedAB && core.A.s_k == 1 && core.B.s_k == 1 && core.K >= 16 && largeB;
-    const bool kmajorWk = kmajor16 || (largeB && lowp16 && core.B.dt == core.computeDt && core.B.s_r == 1 &&
+    const bool kmajorWk = kmajor16 || ((largeB || (core.Batches() > 1 && core.M > 16)) && lowp16 && core.B.dt == core.computeDt && core.B.s_r == 1 &&
                                        core.B.s_k >= core.N && core.B.s_k % 8 == 0 && core.B.bs[0] % 8 == 0 &&
                                        core.B.bs[1] % 8 == 0 && core.B.bs[2] % 8 == 0 && core.N % 8 == 0 &&
                                        !std::getenv("KUDNN_HIP_PACK_KMAJOR"));
@@ -642,6 +642,14 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
                 core.cfg = wk;
             }
         }
+        if (lowp16 && core.M > 16 && core.B.dt == core.computeDt && (chunkedAB || (kmajorWk && chunked(core.A))) &&
+            !kudnn_is_wavek(core.cfg)) {
+            const double packUs = core.K % 64 != 0 ? 5.0 + bytesAB * static_cast<double>(batches) * 2.0 / 4.2e6 : 0.0;
+            const bool pingpong = core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256;
+            if (const int wk = kudnn_wavek_batch_rule(core.M, core.N, core.K, batches, pingpong, packUs)) {
+                core.cfg = wk;
+            }
+        }
     } else {
         core.engine = ENGINE_MFMA_F32;
         // 128 x 128 tiles from one full round of the 256 CUs on, except below 1024 tiles when the last round is at
@@ -695,13 +703,14 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         bool okBf16 = core.computeDt != KUDNN_DT_F32 &&
                       (((f == KUDNN_CFG_BF16_256x256 || f == KUDNN_CFG_BF16_256x128 || f == KUDNN_CFG_BF16_128x128 ||
                          f == KUDNN_CFG_BF16_PINGPONG_256x256) && mfmaOk) ||
-                       (kudnn_is_wavek(f) && (lowp16 || core.B.dt == KUDNN_DT_S8) && (core.M > 16 || weight8 || byRow || !lowp16)) ||
+                       (kudnn_is_wavek(f) && (lowp16 || core.B.dt == KUDNN_DT_S8) && (core.M > 16 || weight8 || byRow || !lowp16) &&
+                        (f != KUDNN_CFG_WAVEK_64x64_W1 || (lowp16 && !weight8 && !byRow))) ||
                        (f == KUDNN_CFG_SKINNY_BF16 && core.M >= 2 && core.M <= 16 && lowp16) ||
                        (f == KUDNN_CFG_GEMV_MULTI_BF16 && core.M >= 2 && core.M <= 8 && lowp16) ||
                        (f == KUDNN_CFG_GEMV_KSPLIT_BF16 && core.M >= 2 && core.M <= 16 && lowp16));
         bool okF32 = core.computeDt == KUDNN_DT_F32 &&
                      (f == KUDNN_CFG_F32_128x128 || f == KUDNN_CFG_F32_64x64 || f == KUDNN_CFG_F32_KSLICE_16x32 ||
-                      (kudnn_is_wavek(f) && (chunkedAB || byRow)));
+                      (kudnn_is_wavek(f) && f != KUDNN_CFG_WAVEK_64x64_W1 && (chunkedAB || byRow)));
         if (okBf16 || okF32) {
             core.cfg = f;
             const bool skinny = f == KUDNN_CFG_SKINNY_BF16 || f == KUDNN_CFG_GEMV_MULTI_BF16 || f == KUDNN_CFG_GEMV_KSPLIT_BF16;
@@ -714,7 +723,8 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
     // k-rows and batches, and 32-bit offsets. The wave-K tiles of 64 and 128 columns do the same with 64-bit addresses.
     const bool wavek = kudnn_is_wavek(core.cfg);
     const bool wide = core.cfg == KUDNN_CFG_WAVEK_32x64 || core.cfg == KUDNN_CFG_WAVEK_64x64 ||
-                      core.cfg == KUDNN_CFG_WAVEK_64x64_W4 || core.cfg == KUDNN_CFG_WAVEK_64x128;
+                      core.cfg == KUDNN_CFG_WAVEK_64x64_W4 || core.cfg == KUDNN_CFG_WAVEK_64x128 ||
+                      core.cfg == KUDNN_CFG_WAVEK_64x64_W1;
     if ((wavek && kmajorWk && wide) ||
         (kmajor16 && core.engine == ENGINE_MFMA_BF16 && core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256 &&
          core.K * core.B.s_k * 2 < (int64_t(1) << 31) &&
@@ -761,6 +771,7 @@ const char *CfgName(int cfg)
         case KUDNN_CFG_WAVEK_64x64: return "mfma_bf16_wavek_64x64";
         case KUDNN_CFG_WAVEK_64x64_W4: return "mfma_bf16_wavek_64x64_2percu";
         case KUDNN_CFG_WAVEK_64x128: return "mfma_bf16_wavek_64x128_w4";
+        case KUDNN_CFG_WAVEK_64x64_W1: return "mfma_bf16_wavek_64x64_w1";
         case KUDNN_CFG_F32_128x128: return "mfma_f32_128x128";
         case KUDNN_CFG_F32_64x64: return "mfma_f32_64x64";
         case KUDNN_CFG_F32_KSLICE_16x32: return "mfma_f32_kslice_16x32";

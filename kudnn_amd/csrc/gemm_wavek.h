@@ -543,6 +543,11 @@ int launch_type(const GemmOperands &op, const EpiParams &ep, int64_t batches, in
         case KUDNN_CFG_WAVEK_64x64: return launch_tile<CT, BT, 64, 64, f16w8 ? 6 : 8>(op, ep, batches, reg, stream);
         case KUDNN_CFG_WAVEK_64x64_W4: return launch_tile<CT, BT, 64, 64, f16w8 ? 3 : 4>(op, ep, batches, reg, stream);
         case KUDNN_CFG_WAVEK_64x128: return launch_tile<CT, BT, 64, 128, 4>(op, ep, batches, reg, stream);
+        case KUDNN_CFG_WAVEK_64x64_W1:
+            if constexpr (CT == BT && (CT == KUDNN_DT_BF16 || CT == KUDNN_DT_F16)) {
+                return reg ? -1 : launch_tile<CT, BT, 64, 64, 1>(op, ep, batches, false, stream);
+            }
+            return -1;
         default: return -1;
     }
 }

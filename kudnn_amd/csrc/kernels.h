@@ -31,8 +31,9 @@ enum {
     KUDNN_CFG_WAVEK_64x64 = 34,    // 8 (8-bit weights of f16: 6)
     KUDNN_CFG_WAVEK_64x64_W4 = 35, // 4 (8-bit weights of f16: 3)
     KUDNN_CFG_WAVEK_64x128 = 36,   // 4
+    KUDNN_CFG_WAVEK_64x64_W1 = 37, // 1: batches of 16-bit products with a short K
 };
-inline bool kudnn_is_wavek(int cfg) { return cfg >= KUDNN_CFG_WAVEK_16x16 && cfg <= KUDNN_CFG_WAVEK_64x128; }
+inline bool kudnn_is_wavek(int cfg) { return cfg >= KUDNN_CFG_WAVEK_16x16 && cfg <= KUDNN_CFG_WAVEK_64x64_W1; }
 
 // Returns 0 on success, -1 if the launch failed or cfg is unknown. `ct` is the operand (compute) type of the 16- and
 // 8-bit kernels: KUDNN_DT_BF16, KUDNN_DT_F16 (f32 accumulation) or KUDNN_DT_S8 (int32 accumulation, integer
@@ -146,8 +147,8 @@ inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, in
     static const Tile kTiles[] = {{KUDNN_CFG_WAVEK_16x16, 16, 16, 8, 11.5, 1.1, 0.25}, {KUDNN_CFG_WAVEK_16x32, 16, 32, 8, 11.6, 1.1, 0.28},
                                   {KUDNN_CFG_WAVEK_32x16, 32, 16, 8, 11.5, 1.1, 0.28}, {KUDNN_CFG_WAVEK_32x32, 32, 32, 8, 11.7, 1.1, 0.32},
                                   {KUDNN_CFG_WAVEK_64x32, 64, 32, 6, 11.3, 1.1, 0.32}, {KUDNN_CFG_WAVEK_32x64, 32, 64, 6, 11.8, 1.1, 0.32},
-                                  {KUDNN_CFG_WAVEK_64x64, 64, 64, 8, 12.6, 1.25, 0.34}, {KUDNN_CFG_WAVEK_64x64_W4, 64, 64, 4, 12.9, 1.1, 0.44},
-                                  {KUDNN_CFG_WAVEK_64x128, 64, 128, 4, 15.5, 1.1, 0.48}};
+                                  {KUDNN_CFG_WAVEK_64x64, 64, 64, 8, 12.6, 1.25, 0.34}, {KUDNN_CFG_WAVEK_64x64_W4, 64, 64, 4, 12.9, 1.1, 0.40},
+                                  {KUDNN_CFG_WAVEK_64x128, 64, 128, 4, 15.5, 1.1, 0.45}};
     const bool f16w8 = weight8 && ct != KUDNN_DT_S8;          // two 128-byte pieces of an A row a k-tile
     const bool f32 = ct == KUDNN_DT_F32;
     const int64_t bk = f32 ? 32 : (weight8 || ct == KUDNN_DT_S8 ? 128 : 64);
@@ -183,6 +184,29 @@ inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, in
         }
     }
     return bestUs < otherUs ? best : 0;
+}
+
+// The same for batches of 16-bit products of at most 256 k (scores of attention heads, say), which spend their time on
+// tiles that start and end. One wave per 64 x 64 tile took 7 us + 2.5 ns a tile + 1 ns a k-tile of it; the ping-pong
+// kernel 3 us + 7.5 us a round of 256 tiles of 256 x 256, which ragged M and N leave partly empty, + 1.9 us a k-tile of
+// it; the 4-wave kernel 4 us + 4.2 us a round of 256 tiles of 128 x 128 + 0.9 us a k-tile. K off the k-tile adds two
+// packs to the last two. Up to 768 tiles, three a CU, four waves share one: 5.6-7 us a call against 7.6-9.2. Measured
+// (bf16, against the other kernel): 63 x (192 x 376 x 80) 31 -> 12 us, 32 x (256 x 256 x 96) 21 -> 7, 64 x (2048 x 128 x
+// 128) 32 -> 26, 20 x (300 x 1000 x 128) 15.4 -> 12.6; 32 x (1024 x 1024 x 128) stays: 44 against 27.
+inline int kudnn_wavek_batch_rule(int64_t M, int64_t N, int64_t K, int64_t batches, bool pingpong, double packUs)
+{
+    const int64_t KT = (K + 63) / 64;
+    if (batches < 2 || KT > 4) {
+        return 0;
+    }
+    const int64_t bm = pingpong ? 256 : 128;
+    const int64_t tiles = (M + 63) / 64 * ((N + 63) / 64) * batches;
+    const double rounds = static_cast<double>(((M + bm - 1) / bm * ((N + bm - 1) / bm) * batches + 255) / 256);
+    const double kt = static_cast<double>(KT);
+    const double other = packUs + (pingpong ? 3.0 + rounds * (7.5 + 1.9 * kt) : 4.0 + rounds * (4.2 + 0.9 * kt));
+    const bool four = tiles <= 768;
+    const double us = four ? 5.3 + 2.5e-3 * static_cast<double>(tiles) : 7.0 + static_cast<double>(tiles) * (2.5e-3 + 1e-3 * kt);
+    return us < other ? (four ? KUDNN_CFG_WAVEK_64x64_W4 : KUDNN_CFG_WAVEK_64x64_W1) : 0;
 }
 int kudnn_launch_gemm_pingpong(const GemmOperands &op, const EpiParams &ep, int64_t batches, int ct, void *ws,
                                bool slicesOk, hipStream_t stream);

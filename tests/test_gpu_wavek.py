@@ -13,7 +13,8 @@ torch = pytest.importorskip("torch")
 
 TILES = {"28": "16x16_w8", "29": "16x32_w8", "30": "32x16_w8", "31": "32x32_w8", "32": "32x64_w6", "33": "64x32_w6", "34": "64x64 ", "35": "64x64_2percu",
          "36": "64x128_w4"}
-WIDE = ("32", "34", "35", "36")  # the tiles that read a [K][N] weight in place
+LOWP = dict(list(TILES.items())[2:], **{"37": "64x64_w1"})  # the tiles of 16-bit operands
+WIDE = ("32", "34", "35", "36", "37")  # the tiles that read a [K][N] weight in place
 ROWS = ("28", "29", "31", "32", "33", "35")  # the tiles that read unaligned rows (from 4 MB of weight on)
 
 
@@ -26,18 +27,18 @@ def gpu():
 
 # K: one chunk, one k-tile, a k-tile and a chunk, fewer k-tiles than waves, one each, one more; odd (packed)
 @pytest.mark.gpu
-@pytest.mark.parametrize("cfg", list(TILES)[2:])
+@pytest.mark.parametrize("cfg", list(LOWP))
 @pytest.mark.parametrize("M,N,Kd", [(17, 16, 8), (32, 33, 64), (33, 130, 72), (64, 128, 320), (65, 264, 512), (70, 40, 584),
                                     (255, 7, 1000), (40, 72, 131)])
 @pytest.mark.parametrize("dt", [O.BF16, O.F16])
 def test_tiles_exact(gpu, monkeypatch, cfg, M, N, Kd, dt):
     monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
     d, _ = run_gemm(T([M, Kd], dt), T([Kd, N], dt, "BA"), T([M, N], dt), T([1, N], O.F32), seed=850, int_valued=True)
-    assert TILES[cfg] in d and ("pack" in d) == (Kd % 8 != 0), d
+    assert LOWP[cfg] in d and ("pack" in d) == (Kd % 8 != 0), d
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("cfg", list(TILES)[2:])
+@pytest.mark.parametrize("cfg", list(LOWP))
 @pytest.mark.parametrize("M,N,Kd", [(17, 8, 64), (64, 128, 448), (70, 200, 512), (130, 264, 64), (33, 72, 200), (33, 70, 128)])
 def test_kmajor_weight_exact(gpu, monkeypatch, cfg, M, N, Kd):
     # [K][N]: in place by the wide tiles when N is a multiple of 8 and K of 64, packed otherwise
@@ -129,7 +130,7 @@ def test_f32_planner_against_float64(gpu):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("cfg", ["30", "35"])
+@pytest.mark.parametrize("cfg", ["30", "35", "37"])
 def test_batches_and_pitches_exact(gpu, monkeypatch, cfg):
     monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
     run_gemm(T([3, 40, 136], O.BF16, "ABC", [40 * 144, 144, 1]), T([3, 136, 72], O.BF16, "ACB"), T([3, 40, 72], O.BF16),
@@ -184,6 +185,16 @@ def test_planner_plans_and_graph_replays(gpu, M, N, Kd, wl):
         assert np.array_equal(from_device(dy, dt), eager)
 
 
+# batches by the planner: a wave a tile, four waves a tile; M, N and K off the tile, both weight layouts
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,M,N,Kd,wl,name", [(20, 300, 1000, 80, "ACB", "64x64_w1"), (20, 300, 1000, 128, "ABC", "64x64_w1"),
+                                              (9, 130, 129, 96, "ACB", "64x64_2percu"), (9, 130, 136, 72, "ABC", "64x64_2percu")])
+def test_short_k_batches_exact(gpu, B, M, N, Kd, wl, name):
+    d, _ = run_gemm(T([B, M, Kd], O.F16), T([B, Kd, N], O.F16, wl), T([B, M, N], O.F16), T([B, 1, N], O.F32), seed=854,
+                    int_valued=True)
+    assert name in d and "pack" not in d, d
+
+
 def test_planner_rule():
     def plan(M, Kd, N, wl="BA", dt=K.BF16):
         return K.LinearPostOps(K.desc([M, Kd], dt), K.desc([Kd, N], dt, wl), K.desc([M, N], dt)).describe()
@@ -197,6 +208,12 @@ def test_planner_rule():
     assert plan(16, 4096, 4096).startswith("skinny") and "wavek" not in plan(256, 4096, 4096)
     assert "wavek" not in plan(16, 4096, 4096) and plan(16, 4097, 4096).startswith("skinny_bf16_wavek_16x")
     assert "wavek" not in plan(255, 4096, 14336) and "wavek" not in plan(40, 128, 4096)
+    def planb(B, M, Kd, N, wl="ACB"):
+        return K.Gemm(K.desc([B, M, Kd], K.BF16), K.desc([B, Kd, N], K.BF16, wl), K.desc([B, M, N], K.BF16)).describe()
+    assert planb(63, 192, 80, 376).startswith("mfma_bf16_wavek_64x64_w1") and "kmajorB" in planb(63, 192, 80, 376, "ABC")
+    assert planb(32, 256, 96, 256).startswith("mfma_bf16_wavek_64x64_2percu")
+    assert "wavek" not in planb(32, 1024, 128, 1024) and "wavek" not in planb(16, 512, 512, 512)
+    assert "skinny" in planb(8, 8, 64, 256) and "wavek_64x64_w1" in planb(16, 128, 128, 2048)
     # 8-bit weights: from M = 1, K of at least 4 k-tiles of 128 (the last may be partial) in whole 16-byte chunks
 
     def plan8(M, Kd, N, adt, bdt, cdt):
