@@ -125,3 +125,35 @@ def test_module_from_linear_fuses_postops():
     torch.cuda.synchronize()
     ref = torch.nn.functional.gelu(x.float() @ lin.weight.float().T + lin.bias.float(), approximate="tanh") + r.float()
     assert torch.allclose(y.float(), ref, rtol=3e-2, atol=3e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lead,stride", [((), None), ((5,), None), ((0,), None), ((2, 3), None), ((6,), "row"), ((2, 3), "t"),
+                                         ((4,), "expand"), ((1,), "row")])
+def test_operand_forms_give_the_dense_result(lead, stride):
+    # x and src of any number of leading dims and any strides, on a side stream, against the call on dense copies
+    g = torch.Generator().manual_seed(12)
+    m, (k, n) = int(np.prod(lead)), (72, 40)
+
+    def form(cols):
+        if stride == "row":  # rows inside wider ones
+            return torch.randn(*lead, cols + 8, generator=g).bfloat16().cuda()[..., :cols]
+        if stride == "t":  # leading dims swapped
+            return torch.randn(*lead[::-1], cols, generator=g).bfloat16().cuda().transpose(0, 1)
+        if stride == "expand":
+            return torch.randn(1, cols, generator=g).bfloat16().cuda().expand(*lead, cols)
+        return torch.randn(*lead, cols, generator=g).bfloat16().cuda()
+    x, src = form(k), form(n)
+    w = torch.randn(k, n, generator=g).bfloat16().cuda().t()
+    b = torch.randn(2 * n, generator=g).bfloat16().cuda()[::2]
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        got = T.linear(x, w, b, act="relu", binary="add", src=src)
+    side.synchronize()
+    assert got.shape == (*lead, n) and got.is_contiguous()
+    if m:
+        ref = T.linear(x.contiguous().view(m, k), w.contiguous(), b.contiguous(), act="relu", binary="add",
+                       src=src.contiguous().view(m, n))
+        torch.cuda.synchronize()
+        assert torch.equal(got.reshape(m, n), ref)
