@@ -1461,8 +1461,8 @@ TensorSpec SpecOf(const kudnn_tensor_desc &d)
 namespace {
 
 // Layout: the split-K arrival counters (KUDNN_SPLIT_MAX_TILES uint32, padded to 512 bytes), then the workspace.
-constexpr size_t kScratchBytes = size_t(64) << 20;
-constexpr size_t kScratchCounterBytes = 512;
+constexpr size_t kScratchBytes = KUDNN_FIXED_BYTES;
+constexpr size_t kScratchCounterBytes = KUDNN_FIXED_COUNTERS;
 static_assert(KUDNN_SPLIT_MAX_TILES * sizeof(uint32_t) <= kScratchCounterBytes, "counter region");
 
 }  // namespace

@@ -59,6 +59,23 @@ void kudnn_pingpong_split(const GemmOperands &op, int64_t batches, int ct, int *
 int kudnn_pingpong_slices(const GemmOperands &op, int64_t batches, int ct);
 // Tiles in slices when only the last partial round is sliced (0: none, or every tile).
 int kudnn_pingpong_slice_tail(const GemmOperands &op, int64_t batches, int ct);
+// Device scratch of the allocation-free entry point: the split-K counters (KUDNN_SPLIT_MAX_TILES uint32), then the
+// workspace.
+constexpr int64_t KUDNN_FIXED_BYTES = int64_t(64) << 20, KUDNN_FIXED_COUNTERS = 512;
+constexpr int64_t KUDNN_FIXED_WORKSPACE = KUDNN_FIXED_BYTES - KUDNN_FIXED_COUNTERS;
+// Whether S slices leave every call of the allocation-free entry point accepted that is accepted unsliced: with no
+// operand packed, either or both (16-bit), what fits the scratch without the sums fits with them.
+inline bool kudnn_slices_fit(int64_t M, int64_t N, int64_t K, int64_t S)
+{
+    const auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
+    const int64_t sums = up(S * M * ((N + 31) / 32 * 32) * 4), a = up(M * K * 2), b = up(N * K * 2);
+    for (const int64_t packs : {int64_t(0), a, b, a + b}) {
+        if (packs <= KUDNN_FIXED_WORKSPACE && packs + sums > KUDNN_FIXED_WORKSPACE) {
+            return false;
+        }
+    }
+    return true;
+}
 // The planner's K-slice count for the ping-pong kernel (0: none) of an M x N grid with KT k-tiles of 128 bytes.
 // Measured on MI355X over 26 shapes (M 256..4096, N 1152..14336, K 2048..14336, against the unsliced ping-pong, its
 // tail split and the 4-wave kernel): up to 64 tiles of 256 x 256, as many slices as keep tiles x slices <= 128 (at
@@ -66,6 +83,12 @@ int kudnn_pingpong_slice_tail(const GemmOperands &op, int64_t batches, int ct);
 // than 64 k-tiles, where the 4-wave kernel's 128 x 128 tiles fill the CUs (2048 x 2048 x 2048: 49 against 38 us);
 // 80-96 tiles with M >= 1024 and at least 48 k-tiles: two slices, 7-23 % faster (M = 512 lost 3 %, 112-128 tiles up
 // to 47 %).
+// 65-120 tiles otherwise: two slices where 9 us + 0.6 us a k-tile (10 % more from 97 tiles on) + the sums' way at 3.6
+// TB/s is 5 % less than 5 us + 1.05 us a k-tile of the whole tiles (1.2 where M is off the tile: edge rows are copied
+// one block at a time). Measured (bf16, unsliced against two slices): 738 x 5896 x 10112 178 -> 110 us, 512 x 11008 x
+// 14336 281 -> 180, 376 x 11840 x 3584 72 -> 62, 768 x 8192 x 8192 140 -> 116; below the line 1100 x 4096 x 2560 50
+// against 54, 700 x 8192 x 2048 48 against 57; 128 tiles fill the chip twice over (2048 x 4096 x 8192 143 against 155).
+// Three slices gained 3 % on two at 72 tiles and lost 35-60 % at 86.
 inline int kudnn_kslice_rule(int64_t M, int64_t N, int64_t KT, int64_t batches, int ct)
 {
     if (batches != 1 || ct == KUDNN_DT_S8 || M <= 0 || N <= 0) {
@@ -82,6 +105,11 @@ inline int kudnn_kslice_rule(int64_t M, int64_t N, int64_t KT, int64_t batches, 
         }
     } else if (tiles <= 96 && M >= 1024 && KT >= 48) {
         S = 2;
+    } else if (tiles <= 120) {
+        const double kt = static_cast<double>(KT), mn = static_cast<double>(M) * static_cast<double>(N);
+        const double whole = 5.0 + (M % 256 != 0 ? 1.2 : 1.05) * kt;
+        const double half = 9.0 + 0.6 * kt * (tiles > 96 ? 1.1 : 1.0) + mn * 16.0 / 3.6e6;
+        S = half * 1.05 < whole && kudnn_slices_fit(M, N, KT * 64, 2) ? 2 : 0;
     }
     return S >= 2 ? static_cast<int>(S) : 0;
 }

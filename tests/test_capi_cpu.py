@@ -205,7 +205,7 @@ def test_f32_kmajor_weight_rule(monkeypatch):
 
 def test_kslice_rule():
     # small 16-bit grids: the ping-pong kernel with K slices (tiles x slices <= 128, slices of >= 16 k-tiles); not at
-    # 64 tiles with < 64 k-tiles (the 4-wave kernel), nor from 97 tiles on, nor for M < 1024 above 64 tiles
+    # 64 tiles with < 64 k-tiles (the 4-wave kernel); two slices of 65-120 tiles where their estimate is the lower one
     for (M, N, Kd), S in {(256, 4096, 4096): 4, (256, 4096, 14336): 8, (512, 4096, 14336): 4, (1024, 4096, 11008): 2,
                           (4096, 1152, 4608): 2, (4096, 1536, 5120): 2}.items():
         d = plan_of(M, Kd, N).describe()

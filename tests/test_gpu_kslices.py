@@ -279,3 +279,31 @@ def test_no_tail_slices_where_they_lose():
     for M, N, Kd in ((4096, 11008, 4096), (2048, 11008, 4096), (4096, 4608, 1152)):
         plan = K.Gemm(K.desc([M, Kd], K.BF16), K.desc([Kd, N], K.BF16, "BA"), K.desc([M, N], K.BF16))
         assert "kslices" not in plan.describe(), plan.describe()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,Kd,wl,dt", [(300, 9001, 4096, "BA", "bf16"), (257, 8457, 4160, "BA", "f16"), (390, 9000, 4096, "AB", "bf16")])
+def test_two_slices_of_65_to_120_tiles_exact(monkeypatch, M, N, Kd, wl, dt):
+    # rows of the sums padded to whole lines, ragged M and N, both layouts; small integers: every sum is exact in f32
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", "4")  # the ping-pong kernel; the slices are the planner's
+    g = torch.Generator(device="cuda").manual_seed(760)
+    kt, tt = (K.BF16, torch.bfloat16) if dt == "bf16" else (K.F16, torch.float16)
+    x = torch.randint(-2, 3, (M, Kd), device="cuda", generator=g).to(tt)
+    w = torch.randint(-2, 3, (N, Kd) if wl == "BA" else (Kd, N), device="cuda", generator=g).to(tt)
+    b = torch.randint(-8, 9, (N,), device="cuda", generator=g).float()
+    y = torch.full((M, N), -1.0, device="cuda", dtype=torch.float32)
+    plan = K.Gemm(K.desc([M, Kd], kt), K.desc([Kd, N], kt, wl), K.desc([M, N], K.F32), K.desc([1, N], K.F32))
+    assert " kslices=2" in plan.describe() and ("kmajorB" in plan.describe()) == (wl == "AB"), plan.describe()
+    plan.run(x, w, y, b)
+    torch.cuda.synchronize()
+    ref = x.float() @ (w.float().t() if wl == "BA" else w.float()) + b
+    assert torch.equal(y, ref)
+
+
+def test_two_slices_rule():
+    def plan(M, Kd, N):
+        return K.LinearPostOps(K.desc([M, Kd], K.BF16), K.desc([Kd, N], K.BF16, "BA"), K.desc([M, N], K.BF16)).describe()
+    assert " kslices=2" in plan(738, 10112, 5896) and " kslices=2" in plan(512, 14336, 11008)
+    assert "kslices" not in plan(700, 2048, 8192) and "kslices" not in plan(2048, 8192, 4096)
+    # the sums and a packed A together exceed the scratch of the allocation-free entry point: stays unsliced
+    assert "kslices" not in plan(768, 11008, 8192)
