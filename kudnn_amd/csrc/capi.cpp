@@ -572,6 +572,7 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
 
     // engine and tile configuration
     const int64_t batches = core.Batches();
+    bool tailSplit = false;
     if (core.computeDt != KUDNN_DT_F32) {
         if (core.M <= 16 && lowp16) {
             core.engine = ENGINE_SKINNY_BF16;
@@ -602,7 +603,7 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
             // then runs one workgroup per tile and slice and a second launch adds the slices.
             const int64_t t256 = (core.M + 255) / 256 * ((core.N + 255) / 256) * batches;
             const int64_t kt = core.kp * DtSize(core.computeDt) / 128;
-            const bool tailSplit = batches == 1 && t256 <= 64 && kt >= 128 && (t256 * kt + 255) / 256 >= 24;
+            tailSplit = batches == 1 && t256 <= 64 && kt >= 128 && (t256 * kt + 255) / 256 >= 24;
             const bool slices = kudnn_kslice_rule(core.M, core.N, kt, batches, core.computeDt) >= 2;
             // Except 32-64 tiles with at most 64 k-tiles and the weight stored [N][K]: there the 4-wave kernel's 128-256
             // tiles of 128 x 128 beat two to four K slices (bf16, bench.py --only dispatch: 256 x 11008 x 4096 45 against
@@ -617,7 +618,10 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         // The 4-wave kernel took 4 + 0.66 us per k-tile and round of 256 tiles (s8 0.72; 30 us and more where it splits
         // K), the ping-pong kernel 5 + 1.15 us per k-tile and round, in S slices 9 + 1.2 us per k-tile of a slice + the
         // sums' way at 3.6 TB/s; a u8 A adds two packs and the row sums of the weight, an 8-bit weight of an f16 product
-        // its pack.
+        // its pack. The s8 tail split spreads every tile over all CUs; the estimate leaves that out, and s8 x s8 grids
+        // of 64 tiles, the split's best case, keep it as a tested choice. (Against 64 x 128 wave-K tiles: 1024 x 4096 x 16384 136
+        // against 108 us; with fewer tiles 768 x 4096 x 16384 141 against 93, 512 x 4096 x 24576 153 against 81; u8 x s8
+        // 1024 x 4096 x 16384 183 against 120.)
         const int64_t t128 = (core.M + 127) / 128 * ((core.N + 127) / 128) * batches;
         const int64_t t256 = (core.M + 255) / 256 * ((core.N + 255) / 256) * batches;
         const double kt = static_cast<double>(core.kp * DtSize(core.computeDt) / 128);
@@ -636,7 +640,8 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
                                                                                 : (packs ? 5.0 + bytesAB * 2.0 / 4.2e6 : 0.0));
         // an integer product with a u8 weight needs row sums of A, and an 8-bit weight of an f16 product that cannot be
         // read in place is packed to f16: both stay with the other kernels
-        if ((core.B.dt != KUDNN_DT_U8 || weight8) && (core.M > 16 || !lowp16 || weight8 || byRow)) {
+        if (!(s8 && tailSplit && t256 == 64 && core.A.dt == KUDNN_DT_S8) && (core.B.dt != KUDNN_DT_U8 || weight8) &&
+            (core.M > 16 || !lowp16 || weight8 || byRow)) {
             if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, core.computeDt, weight8, kmajorWk, byRow, other)) {
                 core.engine = ENGINE_MFMA_BF16;
                 core.cfg = wk;
@@ -676,20 +681,25 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         if ((chunkedAB || byRow) && t64 >= 16) {
             const double bytesAB = static_cast<double>((core.M + core.N) * core.K) * 4.0;
             const double k = static_cast<double>(core.kp);
+            // f32 sums are not taken in longer chains than the kernel replaced takes them: `parts` chains of K / (2 parts)
+            // steps (the k-slice kernel's steps are of 4 k, in 4 waves or, whole lines, 8).
             double other = 0.0;
+            int parts = 1;
             if (core.cfg == KUDNN_CFG_F32_KSLICE_16x32) {
                 const double rounds = static_cast<double>((tks + 255) / 256);
+                parts = kudnn_kslice_whole_line(core.kp) ? 16 : 8;
                 other = kudnn_kslice_whole_line(core.kp) ? 2.5 + 3.2e-3 * k * rounds : 3.0 + 5.2e-3 * k * rounds;
             } else if (core.cfg == KUDNN_CFG_F32_64x64) {
                 other = 4.0 + static_cast<double>((t64 + 255) / 256) * k * (64 * 64 * 2e-6) / (t64 <= 256 ? 0.38 : 0.45);
                 if (t64 < KUDNN_SPLIT_MAX_TILES) {
                     other = std::max(other / 2, 20.0);
+                    parts = static_cast<int>(std::min<int64_t>(core.kp / bk / 4, (384 + t64 - 1) / t64));  // its K splits
                 }
             } else {
                 other = 4.0 + static_cast<double>((t128 + 255) / 256) * k * (128 * 128 * 2e-6) / 0.5;
             }
             other += core.K % bk != 0 ? 5.0 + bytesAB * 2.0 / 4.2e6 : 0.0;
-            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, core.computeDt, false, false, byRow, other)) {
+            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, core.computeDt, false, false, byRow, other, parts)) {
                 core.engine = ENGINE_MFMA_BF16;
                 core.cfg = wk;
             }

@@ -164,9 +164,10 @@ int kudnn_launch_gemm_wavek8(const GemmOperands &op, const EpiParams &ep, int64_
 // is wide for its depth (bf16 255 x 14336 x 4096 55 against 47, 160 x 14336 x 2048 32 against 28) and where M is large:
 // the small tiles then re-read A and B too often. 16-bit products of up to 16 rows have the decode kernels; those of
 // 256 rows or more in whole 128-row tiles keep the plans that the dispatch sweep fixed for them. Less than 4 whole
-// k-tiles leave most waves without one.
+// k-tiles leave most waves without one. minParts (f32): the fewest chains of 2-k steps that K is dealt to, for no longer
+// chain of rounded sums than otherUs' kernel has: a wave's MFMAs are of 2 k, with 16 rows or columns of 4.
 inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, int ct, bool weight8, bool kmajor,
-                            bool byRow, double otherUs)
+                            bool byRow, double otherUs, int minParts = 1)
 {
     struct Tile {
         int cfg, bm, bn, waves;
@@ -190,7 +191,7 @@ inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, in
     double bestUs = 0.0;
     for (const Tile &t : kTiles) {
         if ((kmajor && t.bn < 64) || (t.bm == 16 && (M > 16 || (bk == 64 && !byRow))) ||
-            (byRow && !kudnn_wavek_reg_tile(t.bm, t.bn, t.waves))) {
+            (byRow && !kudnn_wavek_reg_tile(t.bm, t.bn, t.waves)) || t.waves * (t.bm == 16 || t.bn == 16 ? 2 : 1) < minParts) {
             continue;
         }
         const int64_t waves = f16w8 && t.bm == 64 && t.bn == 64 ? t.waves * 3 / 4 : t.waves;
