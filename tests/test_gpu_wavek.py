@@ -229,11 +229,11 @@ def test_planner_rule():
     assert "wavek" in plan(400, 4096, 4096) and "wavek" not in plan(512, 4096, 4096) and "wavek" not in plan(1000, 4096, 11008)
     def plan32(M, Kd, N):
         return K.Gemm(K.desc([M, Kd], K.F32), K.desc([Kd, N], K.F32, "BA"), K.desc([M, N], K.F32)).describe()
-    # f32: as many chains as the k-slice kernel (8 or 16) or the split grid has; a whole-line K leaves 32 x 16 only
-    assert plan32(240, 1298, 1400).startswith("mfma_f32_kslice_32x32_w8") and "_16x32" in plan32(200, 1023, 1400)
+    # f32: chains of sums half as long as the k-slice kernel's or the split grid's leave 32 x 16 tiles, rows of whole chunks
+    assert plan32(64, 2000, 2000).startswith("mfma_f32_kslice_32x16_w8") and "_16x32" in plan32(200, 1023, 1400)
     assert "_64x128_w4" in plan32(500, 3000, 3000)
     # s8: 64 tiles of 256 x 256 and 128 k-tiles or more keep the tail split, fewer tiles and u8 sources do not
     assert "pingpong" in plan8(1024, 16384, 4096, K.S8, K.S8, K.S32) and "wavek" in plan8(768, 16384, 4096, K.S8, K.S8, K.S32)
     assert "wavek" in plan8(1024, 16384, 4096, K.U8, K.S8, K.S32)
-    assert plan32(107, 2176, 1984).startswith("mfma_f32_kslice_32x") and "pack" not in plan32(240, 1298, 1400)
+    assert plan32(107, 2176, 1984).startswith("mfma_f32_kslice_32x") and "_16x32" in plan32(240, 1298, 1400)
     assert plan32(128, 1024, 1024).startswith("mfma_f32_kslice_16x32") and plan32(2048, 4096, 4096).startswith("mfma_f32_128x128")
