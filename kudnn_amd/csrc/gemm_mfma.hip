@@ -469,24 +469,27 @@ __global__ __launch_bounds__(WM *WN * 64, 1) void gemm_mfma_kernel(GemmOperands 
                 }
             }
         } else if constexpr (FORM == EPI_FORM_GENERIC) {
+            // Runs of 8 columns, then, in a loop of its own, the elements that they leave (no vec8, or a row's last run).
+            // Against both forms in one loop over all columns: 8192 x 1 x 256 bf16 11.2 us (15.3), a transposed bf16
+            // output of 2048 x 2048 x 1024 45 us (47), a transposed f32 one with a residual 59 (57).
+            const int64_t mW = m0 + wm * TM;
+            if (ep.vec8) {
 #pragma unroll 1
-            for (int r = lane >> 2; r < TM; r += 16) {
-                const int64_t m = m0 + wm * TM + r;
-                if (m >= M) {
-                    continue;
-                }
-                const float *src = stage + r * kStagePitch + col8;
-                if (ep.vec8 && n + 7 < N) {
+                for (int r = lane >> 2; r < TM && mW + r < M && n + 7 < N; r += 16) {
+                    const float *src = stage + r * kStagePitch + col8;
                     const float4 lo = *reinterpret_cast<const float4 *>(src);
                     const float4 hi = *reinterpret_cast<const float4 *>(src + 4);
                     const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-                    epi_apply8(ep, ob, m, n, v);
-                    continue;
+                    epi_apply8(ep, ob, mW + r, n, v);
                 }
+            }
+            if (!ep.vec8 || n - col8 + 32 > N) {
+                const int cols = ep.vec8 && n + 7 < N ? 0 : (n + 8 <= N ? 8 : static_cast<int>(N - n));
 #pragma unroll 1
-                for (int q = 0; q < 8; ++q) {
-                    if (n + q < N) {
-                        epi_apply(ep, ob, m, n + q, src[q]);
+                for (int r = lane >> 2; r < TM && mW + r < M; r += 16) {
+#pragma unroll 1
+                    for (int q = 0; q < cols; ++q) {
+                        epi_apply(ep, ob, mW + r, n + q, stage[r * kStagePitch + col8 + q]);
                     }
                 }
             }

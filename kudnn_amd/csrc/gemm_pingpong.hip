@@ -322,8 +322,11 @@ __device__ __forceinline__ void epilogue_edge(const EpiParams &ep, const EpiBatc
 }
 
 // Epilogue of any tile in the generic form (activation and tensor types read at run time): runs of 8 columns where the
-// host allows it (vec8), else one element at a time. The strips are a rolled loop with one copy of the epilogue's code;
-// only the staging, which must name its accumulators, is unrolled.
+// host allows it (vec8), one element at a time otherwise and in the last, partial run of a row, each in a loop of its own.
+// The strips are a rolled loop with one copy of the epilogue's code; only the staging, which must name its accumulators,
+// is unrolled. Strips, rows and columns past the matrix are not walked: 20480 x 1 x 128 bf16, one column of 80 tiles, takes
+// 12 us a call (walking them all, with both forms in one loop, 34; before there were runs, 21), and 165504 x 1 x 40 45 us
+// (120; 85).
 __device__ __forceinline__ void epilogue_generic(const EpiParams &ep, const EpiBatch &ob, const f32x16_t (&acc)[4][2],
                                                  float *stage, int lane, int64_t mW, int64_t nW, int64_t M, int64_t N)
 {
@@ -331,7 +334,7 @@ __device__ __forceinline__ void epilogue_generic(const EpiParams &ep, const EpiB
     const int col8 = (lane & 3) * 8, rl = lane >> 2;
     __syncthreads();  // every wave is done with the tile buffers that the staging area reuses
 #pragma unroll 1
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < 4 && nW + j * 32 < N; ++j) {
         const int64_t n = nW + j * 32 + col8;
         sfor<4>([&](auto jc) __attribute__((always_inline)) {
             if (j == decltype(jc)::value) {
@@ -341,22 +344,24 @@ __device__ __forceinline__ void epilogue_generic(const EpiParams &ep, const EpiB
             }
         });
         wave_sync();
+        if (ep.vec8) {
 #pragma unroll 1
-        for (int ps = 0; ps < 4; ++ps) {
-            const int r = rl + ps * 16;
-            const int64_t m = mW + r;
-            const float *src = stage + r * kPitch + col8;
-            if (m < M && ep.vec8 && n + 7 < N) {
+            for (int r = rl; r < 64 && mW + r < M && n + 7 < N; r += 16) {
+                const float *src = stage + r * kPitch + col8;
                 const float4 lo = *reinterpret_cast<const float4 *>(src);
                 const float4 hi = *reinterpret_cast<const float4 *>(src + 4);
                 const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-                epi_apply8(ep, ob, m, n, v);
-            } else if (m < M) {
+                epi_apply8(ep, ob, mW + r, n, v);
+            }
+        }
+        if (!ep.vec8 || nW + j * 32 + 32 > N) {
+            // columns n .. of this lane that the loop above left
+            const int cols = ep.vec8 && n + 7 < N ? 0 : (n + 8 <= N ? 8 : static_cast<int>(N - n));
 #pragma unroll 1
-                for (int q = 0; q < 8; ++q) {
-                    if (n + q < N) {
-                        epi_apply(ep, ob, m, n + q, src[q]);
-                    }
+            for (int r = rl; r < 64 && mW + r < M; r += 16) {
+#pragma unroll 1
+                for (int q = 0; q < cols; ++q) {
+                    epi_apply(ep, ob, mW + r, n + q, stage[r * kPitch + col8 + q]);
                 }
             }
         }

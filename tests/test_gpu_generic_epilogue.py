@@ -78,3 +78,54 @@ def test_integer_runs(M, N, Kd, adt, bdt, bias):
     ref = c.clone_empty()
     O.gemm(x.t, w.t, ref, b.t if b else None)
     assert np.array_equal(from_device(dc, O.S32), ref.buf), plan.describe()
+
+
+@pytest.mark.parametrize("kernel", list(KERNELS))
+@pytest.mark.parametrize("M,N", [(257, 1), (70, 2), (300, 9), (65, 33), (257, 264)])
+@pytest.mark.parametrize("ylayout", ["AB", "BA"])
+def test_few_columns_and_transposed(monkeypatch, kernel, M, N, ylayout):
+    # the element-wise loop alone (no run of 8 columns fits, or the output's columns are not contiguous) and after the runs,
+    # with strips of a wave's tile past the matrix
+    cfg, slices = KERNELS[kernel]
+    monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
+    if slices is not None:
+        monkeypatch.setenv("KUDNN_HIP_FORCE_KSLICES", slices)
+    dt, Kd = (O.F32, 64) if kernel == "f32" else (O.F16 if kernel == "four_wave" else O.BF16, 128)
+    x = Case([M, Kd], dt, seed=840, dist="normal", lo=0.0, hi=1.0)
+    w = Case([Kd, N], dt, "BA", seed=841, dist="normal", lo=0.0, hi=0.1)
+    b = Case([1, N], O.F32, seed=842, lo=-0.2, hi=0.2)
+    y = Case([M, N], dt, ylayout, zero=True)
+    plan = K.Gemm(x.desc, w.desc, y.desc, b.desc)
+    dy = zeros_device(y)
+    plan.run(x.device(), w.device(), dy, b.device(), alpha=0.5)
+    torch.cuda.synchronize()
+    ref = y.clone_empty()
+    O.gemm(x.t, w.t, ref, b.t, 0.5)
+    compare(from_device(dy, dt), ref.buf, dt, plan.describe())
+
+
+def test_one_column_is_not_slower_than_a_tile():
+    # 20480 x N x 128 takes the same 80 tiles for N = 1 and N = 128. Walking every strip and column of a tile for one
+    # column made N = 1 2.2 times as long as N = 128 (33.7 against 15.4 us); half of it is left as the margin
+    M, Kd, us = 20480, 128, {}
+    x = torch.randn(M, Kd, device="cuda").bfloat16()
+    for N in (1, 128):
+        w, y = torch.randn(N, Kd, device="cuda").bfloat16(), torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+        plan = K.Gemm(K.desc([M, Kd], K.BF16), K.desc([Kd, N], K.BF16, "BA"), K.desc([M, N], K.BF16))
+        assert "pingpong" in plan.describe() and "pack" not in plan.describe(), plan.describe()
+        plan.run(x, w, y)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                plan.run(x, w, y, stream=torch.cuda.current_stream())
+        t = []
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            graph.replay()
+            e1.record()
+            torch.cuda.synchronize()
+            t.append(e0.elapsed_time(e1) * 1000 / 20)
+        us[N] = min(t)
+    assert us[1] < 1.6 * us[128], us
