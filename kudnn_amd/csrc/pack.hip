@@ -113,19 +113,22 @@ __device__ __forceinline__ int64_t batch_off(const PackArgs &p, int64_t b)
 
 // Source contiguous along K. A workgroup of 4 waves takes 16 rows x 64 chunks of 16 packed bytes: wave w's lane l
 // converts chunk l of rows w, w + 4, w + 8, w + 12, all four loads issued before the first store. A call of M = 4 on an
-// s8 weight of 4096 x 4096 (f16 x s8: 16.8 MB read, 33.6 MB written) takes 21.5 us, 36.1 one element at a time.
-constexpr int kRowsPerGroup = 16;
+// s8 weight of 4096 x 4096 (f16 x s8: 16.8 MB read, 33.6 MB written) takes 21.5 us, 36.1 one element at a time. Packed
+// rows of at most 32 chunks share a wave, 2^laneBits lanes to a row (a row of one k-tile is 8 chunks: with a wave each,
+// 56 lanes of 64 did nothing: 165504 x 256 x 40 bf16, which packs its source, 59 us a call, 48 this way).
+constexpr int kRowsPerGroup = 16;  // with a wave to a row
 
 template <int SRC, int DST>
-__global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p)
+__global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p, int laneBits)
 {
     using S = Elem<SRC>;
     using D = Elem<DST>;
     constexpr int EPC = 16 / static_cast<int>(sizeof(D));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int chunk = threadIdx.x & ((1 << laneBits) - 1);
+    const int step = 256 >> laneBits;  // rows a workgroup takes at a time
     const int64_t b = blockIdx.z;
-    const int64_t k = (static_cast<int64_t>(blockIdx.y) * 64 + lane) * EPC;
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kRowsPerGroup + wave;
+    const int64_t k = ((static_cast<int64_t>(blockIdx.y) << laneBits) + chunk) * EPC;
+    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * (kRowsPerGroup / 4 * step) + (threadIdx.x >> laneBits);
     if (k >= p.kp) {
         return;  // no barrier below
     }
@@ -139,12 +142,12 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p)
         Vec<S, EPC> in[kRowsPerGroup / 4];
 #pragma unroll
         for (int i = 0; i < kRowsPerGroup / 4; ++i) {
-            const int64_t r = r0 + 4 * i;
+            const int64_t r = r0 + step * i;
             in[i] = *reinterpret_cast<const Vec<S, EPC> *>(src + (r < p.rows ? r : p.rows - 1) * p.s_r);
         }
 #pragma unroll
         for (int i = 0; i < kRowsPerGroup / 4; ++i) {
-            const int64_t r = r0 + 4 * i;
+            const int64_t r = r0 + step * i;
             if (r < p.rows) {
                 Chunk c;
 #pragma unroll
@@ -155,7 +158,7 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p)
         return;
     }
     // the chunk that column K ends in, and the padding after it
-    for (int64_t r = r0; r < p.rows && r < r0 + kRowsPerGroup; r += 4) {
+    for (int64_t r = r0; r < p.rows && r < r0 + kRowsPerGroup / 4 * step; r += step) {
         Chunk c;
 #pragma unroll
         for (int e = 0; e < EPC; ++e) c.e[e] = k + e < p.cols ? convert<SRC, DST>(src[r * p.s_r + e]) : D(0);
@@ -261,9 +264,14 @@ void launch_vector(const PackArgs &p, int64_t batches, hipStream_t stream)
 {
     constexpr int EPC = 16 / static_cast<int>(sizeof(Elem<DST>));
     if (p.s_k == 1) {
-        const dim3 grid(static_cast<unsigned>((p.rows + kRowsPerGroup - 1) / kRowsPerGroup),
-                        static_cast<unsigned>((p.kp + 64 * EPC - 1) / (64 * EPC)), static_cast<unsigned>(batches));
-        hipLaunchKernelGGL((pack_rows_kernel<SRC, DST>), grid, dim3(256), 0, stream, p);
+        int laneBits = 3;  // the fewest lanes that hold a packed row, up to a wave
+        while (laneBits < 6 && (int64_t(EPC) << laneBits) < p.kp) {
+            ++laneBits;
+        }
+        const int64_t rows = kRowsPerGroup / 4 * (256 >> laneBits), k = int64_t(EPC) << laneBits;
+        const dim3 grid(static_cast<unsigned>((p.rows + rows - 1) / rows), static_cast<unsigned>((p.kp + k - 1) / k),
+                        static_cast<unsigned>(batches));
+        hipLaunchKernelGGL((pack_rows_kernel<SRC, DST>), grid, dim3(256), 0, stream, p, laneBits);
     } else {
         const dim3 grid(static_cast<unsigned>((p.rows + kTile - 1) / kTile),
                         static_cast<unsigned>((p.kp + kTile - 1) / kTile), static_cast<unsigned>(batches));

@@ -56,3 +56,16 @@ def test_unaligned_base_pointers(M, N, Kd, shift):
     O.gemm(O.Tensor((M, Kd), (Kd, 1), O.BF16, O.from_f32_rne(xv, O.BF16)),
            O.Tensor((Kd, N), (1, Kd), O.BF16, O.from_f32_rne(wv, O.BF16)), ref)
     assert np.array_equal(from_device(y, O.F32), ref.buf), plan.describe()
+
+
+# packed rows of 1 to 5 k-tiles (8, 16, 24, 32 and 40 chunks of 16 bytes: 8 to 64 lanes to a row), rows off a workgroup's
+@pytest.mark.parametrize("adt,bdt,cdt", [(O.BF16, O.BF16, O.F32), (O.F16, O.S8, O.F32), (O.U8, O.S8, O.S32), (O.BF16, O.F32, O.F32)])
+@pytest.mark.parametrize("rows", [1, 15, 129, 515])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 4, 5])
+def test_narrow_rows_exact(adt, bdt, cdt, rows, tiles):
+    step = 32 if O.F32 in (adt, bdt) else (128 if cdt == O.S32 else 64)
+    for Kd in (tiles * step - 1, (tiles - 1) * step + 3):
+        if bdt == O.S8 and cdt == O.F32:
+            Kd = min(Kd, 199)  # terms of at most 16 x 125: below 2^24
+        d, _ = run_gemm(T([rows, Kd], adt), T([Kd, 24], bdt, "BA"), T([rows, 24], cdt), None, seed=805, int_valued=True)
+        assert "pack" in d, d
