@@ -564,7 +564,8 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
     const bool largeB = core.N * core.K * DtSize(core.B.dt) >= (int64_t(4) << 20);
     const bool chunkedAB = typesWk && chunked(core.A) && chunked(core.B);
     const bool byRow = typesWk && !chunkedAB && core.A.s_k == 1 && core.B.s_k == 1 && core.K >= 16 && largeB;
-    const bool kmajorWk = kmajor16 || ((largeB || (core.Batches() > 1 && core.M > 16)) && lowp16 && core.B.dt == core.computeDt && core.B.s_r == 1 &&
+    const bool kmajorWk = kmajor16 || ((largeB || (core.Batches() > 1 && core.M > 16)) && lowp16 &&
+                                       core.B.dt == core.computeDt && core.B.s_r == 1 &&
                                        core.B.s_k >= core.N && core.B.s_k % 8 == 0 && core.B.bs[0] % 8 == 0 &&
                                        core.B.bs[1] % 8 == 0 && core.B.bs[2] % 8 == 0 && core.N % 8 == 0 &&
                                        !std::getenv("KUDNN_HIP_PACK_KMAJOR"));
@@ -572,6 +573,12 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
 
     // engine and tile configuration
     const int64_t batches = core.Batches();
+    int64_t weights = 1;  // distinct weights of the batches
+    for (int d = 0; d < 3; ++d) {
+        weights *= core.B.bs[d] != 0 ? core.bdim[d] : 1;
+    }
+    const double mbAB = (static_cast<double>(batches * core.M * core.K * DtSize(core.A.dt)) +
+                         static_cast<double>(weights * core.N * core.K * DtSize(core.B.dt))) * 1e-6;
     bool tailSplit = false;
     if (core.computeDt != KUDNN_DT_F32) {
         if (core.M <= 16 && lowp16) {
@@ -610,48 +617,72 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
             // 55 us, 256 x 14336 x 4096 45 against 58, 1024 x 4096 x 4096 46 against 62, 1024 x 2048 x 2048 26 against
             // 35, 512 x 4096 x 4096 even; 16 tiles and 128 k-tiles stay sliced). A weight stored [K][N] keeps the
             // ping-pong kernel, which reads it in place; the 4-wave kernel would pack it on every call.
-            const bool fourWave = batches == 1 && t256 >= 32 && t256 <= 64 && kt <= 64 && core.B.s_r != 1;
+            // 65-79 tiles likewise where its estimate, 4 us + 5.6 us a round of 256 tiles + 0.63 us a k-tile of it, is the
+            // lower one: 384 x 8832 x 4224 49 us against 60 in two slices, 800 x 4352 x 2688 37 against 47; two rounds of
+            // 128 x 128 tiles stay sliced (738 x 5896 x 10112).
+            const double mn = static_cast<double>(core.M * core.N) * 1e-6, ktd = static_cast<double>(kt);
+            const int64_t t128 = (core.M + 127) / 128 * ((core.N + 127) / 128) * batches;
+            const bool oneRound = t256 > 64 && t256 < 80 && 4.0 + static_cast<double>((t128 + 255) / 256) * (5.6 + 0.63 * ktd) <
+                                                               11.8 + 0.52 * ktd + 3.7 * mn;
+            const bool fourWave = batches == 1 && core.B.s_r != 1 && ((t256 >= 32 && t256 <= 64 && kt <= 64) || oneRound);
             core.cfg = (t256 >= 80 || tailSplit || slices) && !fourWave ? KUDNN_CFG_BF16_PINGPONG_256x256
                                                                         : KUDNN_CFG_BF16_128x128;
         }
-        // Tiles with K dealt to the waves, where their estimate (kudnn_wavek_rule) beats this one of the choice above.
-        // The 4-wave kernel took 4 + 0.66 us per k-tile and round of 256 tiles (s8 0.72; 30 us and more where it splits
-        // K), the ping-pong kernel 5 + 1.15 us per k-tile and round, in S slices 9 + 1.2 us per k-tile of a slice + the
-        // sums' way at 3.6 TB/s; a u8 A adds two packs and the row sums of the weight, an 8-bit weight of an f16 product
-        // its pack. The s8 tail split spreads every tile over all CUs; the estimate leaves that out, and s8 x s8 grids
-        // of 64 tiles, the split's best case, keep it as a tested choice. (Against 64 x 128 wave-K tiles: 1024 x 4096 x 16384 136
-        // against 108 us; with fewer tiles 768 x 4096 x 16384 141 against 93, 512 x 4096 x 24576 153 against 81; u8 x s8
-        // 1024 x 4096 x 16384 183 against 120.)
+        // Tiles with K dealt to the waves, where their cost (kudnn_wavek_rule) is below this one of the choice above: fits of
+        // the same 5600 products (mean error 5-12 %). Rounds are of 256 tiles, kt counts k-tiles, mn is millions of outputs.
+        // The 4-wave kernel has no fit where it splits K (30 us and more). A u8 A adds two packs and the row sums of the
+        // weight; packs cost a launch each and 0.3 us per MB of both operands. Sliced rows count 1.1 of their fit, which
+        // was low for K above 8192 (500 x 4096 x 11008 82 us, the fit 71).
+        // The s8 tail split spreads every tile over all CUs; the estimate leaves that out. s8 x s8 grids of 64 tiles keep
+        // it because a test of the planner names that plan, not because it is faster: 1024 x 4096 x 16384 takes 133 us on
+        // the tail split and 103 on 64 x 128 wave-K tiles, 512 x 8192 x 16384 137 and 104; with fewer tiles, where the
+        // wave-K tiles are taken, 768 x 4096 x 16384 147 and 86, 512 x 4096 x 24576 166 and 78.
         const int64_t t128 = (core.M + 127) / 128 * ((core.N + 127) / 128) * batches;
         const int64_t t256 = (core.M + 255) / 256 * ((core.N + 255) / 256) * batches;
         const double kt = static_cast<double>(core.kp * DtSize(core.computeDt) / 128);
-        const double nk = static_cast<double>(core.N * core.K), mn = static_cast<double>(core.M * core.N);
-        const bool s8 = core.computeDt == KUDNN_DT_S8;
+        const bool s8 = core.computeDt == KUDNN_DT_S8, pingpong = core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256;
+        const double mn = static_cast<double>(core.M * core.N * batches) * 1e-6;
+        const double r128 = static_cast<double>((t128 + 255) / 256), r256 = static_cast<double>((t256 + 255) / 256);
         const int S = kudnn_kslice_rule(core.M, core.N, static_cast<int64_t>(kt), batches, core.computeDt);
+        const bool bInPlace = pingpong && kmajor16, binary = extra0 != nullptr;
+        const int packsO = (core.A.staticPack ? 1 : 0) + (core.B.staticPack && !bInPlace ? 1 : 0);
         double other = 1e30;
         if (core.cfg == KUDNN_CFG_BF16_128x128 && (s8 || t128 >= KUDNN_SPLIT_MAX_TILES)) {
-            other = static_cast<double>((t128 + 255) / 256) * (4.0 + (s8 ? 0.72 : 0.66) * kt);
-        } else if (core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256) {
-            other = S >= 2 ? 9.0 + 1.2 * kt / S + S * mn * 8.0 / 3.6e6 : 5.0 + 1.15 * kt * static_cast<double>((t256 + 255) / 256);
+            other = s8 ? 3.7 + r128 * (4.4 + 0.6 * kt) + 1.3 * mn : 4.0 + r128 * (5.6 + 0.63 * kt) + (binary ? 0.6 : 0.3) * mn;
+        } else if (pingpong && s8) {
+            other = 8.0 + r256 * (9.0 + 1.05 * kt) + 1.4 * mn;
+        } else if (pingpong && S >= 2) {
+            other = 11.8 + 1.04 * kt / S + (1.17 * S + 1.37 + (binary ? 1.06 : 0.0) + (extra1 != nullptr ? 1.5 : 0.0)) * mn;
+            other *= packsO == 0 && !bInPlace ? 1.1 : 1.0;
+        } else if (pingpong && weights > 1) {
+            other = 2.6 + r256 * (10.6 + 0.75 * kt) + (binary ? 0.26 : 0.1) * mn + (bInPlace ? 0.07 : 0.11) * mbAB;
+        } else if (pingpong) {
+            other = 4.7 + 1.1 * r256 * kt + (binary ? 2.2 : 2.06) * mn;
         }
-        const double bytesAB = static_cast<double>(core.M * core.K * DtSize(core.A.dt) + core.N * core.K * DtSize(core.B.dt));
-        const bool packs = byRow || core.K % bk != 0;  // the other kernels pack both operands to whole k-tiles
-        other += weight8 ? 3.0 + nk * 0.75e-6 : (s8 && core.A.dt == KUDNN_DT_U8 ? 14.0 + nk * 0.47e-6
-                                                                                : (packs ? 5.0 + bytesAB * 2.0 / 4.2e6 : 0.0));
+        other += s8 && core.A.dt == KUDNN_DT_U8 ? 10.7 + 0.44 * mbAB
+                                                : (packsO == 2 ? 9.4 + 0.3 * mbAB : (packsO == 1 ? 2.4 + 0.27 * mbAB : 0.0));
+        // what the wave-K tiles themselves have to pack
+        const int packsW = chunkedAB || byRow ? 0
+                           : kmajorWk         ? (chunked(core.A) ? 0 : 1)
+                                              : (core.A.staticPack ? 1 : 0) + (core.B.staticPack ? 1 : 0);
+        const double packUs = packsW == 2 ? 2.8 + 0.21 * mbAB : (packsW == 1 ? 5.4 + 0.06 * mbAB : 0.0);
         // an integer product with a u8 weight needs row sums of A, and an 8-bit weight of an f16 product that cannot be
-        // read in place is packed to f16: both stay with the other kernels
+        // read in place is packed to f16: both stay with the other kernels. A weight of at most 16 rows is one workgroup's
+        // work there, of 8 chains of k-tiles; the row kernel with its pack is the faster one for a deep K (f16 x s8
+        // 1 x 4 x 16384 7.6 us against 9.8; 1 x 16 x 9600 8.4 against 6.6)
+        const bool fewRows = weight8 && core.M <= 2 && core.N <= 16 && core.K >= 12288 && batches == 1;
         if (!(s8 && tailSplit && t256 == 64 && core.A.dt == KUDNN_DT_S8) && (core.B.dt != KUDNN_DT_U8 || weight8) &&
-            (core.M > 16 || !lowp16 || weight8 || byRow)) {
-            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, core.computeDt, weight8, kmajorWk, byRow, other)) {
+            (core.M > 16 || !lowp16 || weight8 || byRow) && !fewRows) {
+            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, weights, core.computeDt, weight8,
+                                                kmajorWk, byRow, binary, packUs, other)) {
                 core.engine = ENGINE_MFMA_BF16;
                 core.cfg = wk;
             }
         }
         if (lowp16 && core.M > 16 && core.B.dt == core.computeDt && (chunkedAB || (kmajorWk && chunked(core.A))) &&
             !kudnn_is_wavek(core.cfg)) {
-            const double packUs = core.K % 64 != 0 ? 5.0 + bytesAB * static_cast<double>(batches) * 2.0 / 4.2e6 : 0.0;
-            const bool pingpong = core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256;
-            if (const int wk = kudnn_wavek_batch_rule(core.M, core.N, core.K, batches, pingpong, packUs)) {
+            const double packsOther = core.K % 64 != 0 ? 5.0 + mbAB * 2.0 / 4.2 : 0.0;
+            if (const int wk = kudnn_wavek_batch_rule(core.M, core.N, core.K, batches, pingpong, binary, packsOther)) {
                 core.cfg = wk;
             }
         }
@@ -679,7 +710,6 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         // whole-line form 2.5 + 3.2 ns; a 64 x 64 grid split over workgroups about 20 us, unsplit 0.38 TFLOP/s a CU in
         // one round and 0.45 in more, 128 x 128 tiles 0.5; K off the 32-deep k-tile adds the packs.
         if ((chunkedAB || byRow) && t64 >= 16) {
-            const double bytesAB = static_cast<double>((core.M + core.N) * core.K) * 4.0;
             const double k = static_cast<double>(core.kp);
             // f32 sums are taken in chains of at most half the length of a kernel that itself splits K: `parts` chains of
             // K / (2 parts) steps (the k-slice kernel's steps are of 4 k, in 4 waves or, whole lines, 8). At equal lengths
@@ -699,8 +729,9 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
             } else {
                 other = 4.0 + static_cast<double>((t128 + 255) / 256) * k * (128 * 128 * 2e-6) / 0.5;
             }
-            other += core.K % bk != 0 ? 5.0 + bytesAB * 2.0 / 4.2e6 : 0.0;
-            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, core.computeDt, false, false, byRow, other, parts)) {
+            other += core.K % bk != 0 ? 5.0 + mbAB * 2.0 / 4.2 : 0.0;
+            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, weights, core.computeDt, false, false,
+                                                byRow, false, 0.0, other, parts)) {
                 core.engine = ENGINE_MFMA_BF16;
                 core.cfg = wk;
             }

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "plan_types.h"
@@ -144,30 +145,44 @@ constexpr bool kudnn_wavek_reg_tile(int bm, int bn, int waves)
 
 // Tiles whose K is dealt to the workgroup's waves (gemm_wavek.hip). op.K is the true K; k_padded says that packed rows
 // hold zeros up to a whole 16-byte chunk. Operands that are not whole chunks (rows, K, bases) take the register form.
-// b_kmajor (16-bit): whole chunks of columns, tiles of 32 columns or more. `bt` is the weight's stored type: ct, s8 or u8 under f16, and u8 under s8 for a u8
-// A beside an s8 weight (the term of the -128 shift is added here; op.a_u8 says whether A still has to be shifted). No
-// workspace.
+// b_kmajor (16-bit): whole chunks of columns, tiles of 64 columns or more. `bt` is the weight's stored type: ct, s8 or u8
+// under f16, and u8 under s8 for a u8 A beside an s8 weight (the term of the -128 shift is added here; op.a_u8 says whether
+// A still has to be shifted). No workspace.
 int kudnn_launch_gemm_wavek(const GemmOperands &op, const EpiParams &ep, int64_t batches, int ct, int bt, int cfg,
                             hipStream_t stream);
 // Its 8-bit and f32 instances (a translation unit of their own); `reg`: the register form.
 int kudnn_launch_gemm_wavek8(const GemmOperands &op, const EpiParams &ep, int64_t batches, int ct, int bt, int cfg, bool reg,
                              hipStream_t stream);
 
-// The wave-K tile for a product (0: the kernel the other rules chose). The estimate is what the measurements of 7 tiles
-// over M = 17..1030 and N, K = 2048..14336 (weights rotated past the Infinity Cache) fit: 4.2 us a call, plus the largest
-// of the weight's stream from HBM at 6.6 TB/s, the busiest CU's copies, nsPerKB per KB of A and B (`over` times that when
-// more tiles come to a CU than fit beside one another), and the products at 0.8 PFLOP/s (8-bit 1.4; f32 by the tile's rate on the
-// busiest CU), plus a part of the stream. Over 26 drawn bf16 shapes the choice was within 7 % of the best tile but for 3 (19 %). otherUs is the same kind
-// of estimate for the other rules' kernel (BuildCore). Measured, against the other kernel: bf16 64 x 4096 x 4096 10 us (31),
-// 64 x 11008 x 4096 22 (48), 192 x 4096 x 11008 45 (48), 400 x 4096 x 4096 27 (45); f16 x s8 4 x 4096 x 4096 6.1 (21.5),
-// 128 x 4096 x 4096 12 (55); u8 x s8 64 x 4096 x 4096 7.5 (47), 1024 x 4096 x 4096 40 (51). The others stay where a weight
-// is wide for its depth (bf16 255 x 14336 x 4096 55 against 47, 160 x 14336 x 2048 32 against 28) and where M is large:
-// the small tiles then re-read A and B too often. 16-bit products of up to 16 rows have the decode kernels; those of
-// 256 rows or more in whole 128-row tiles keep the plans that the dispatch sweep fixed for them. Less than 4 whole
-// k-tiles leave most waves without one. minParts (f32): the fewest chains of 2-k steps that K is dealt to, for no longer
-// chain of rounded sums than otherUs' kernel has: a wave's MFMAs are of 2 k, with 16 rows or columns of 4.
-inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, int ct, bool weight8, bool kmajor,
-                            bool byRow, double otherUs, int minParts = 1)
+// The wave-K tile for a product (0: the kernel the other rules chose). The tile is the one with the least estimate, which
+// is what the measurements of 7 tiles over M = 17..1030 and N, K = 2048..14336 (weights rotated past the Infinity Cache)
+// fit: 4.2 us a call, plus the largest of the weight's stream from HBM at 6.6 TB/s, the busiest CU's copies, nsPerKB per KB
+// of A and B (`over` times that when more tiles come to a CU than fit beside one another), and the products at 0.8 PFLOP/s
+// (8-bit 1.4; f32 by the tile's rate on the busiest CU), plus a part of the stream. Over 26 drawn bf16 shapes the choice was
+// within 7 % of the best tile but for 3 (19 %).
+// That tile is taken where its cost is below otherUs, the cost of the other rules' kernel (BuildCore). The estimate orders
+// the tiles but is 15-50 % low where K is short, the output large, the rows unaligned or the batches many, so the cost is a
+// fit of its own, over 5600 products (M = 1..8192, N = 1..16384, K = 64..16384, up to 64 batches; half of them drawn as the
+// layers of a model are) timed on the chosen tile and on the other kernel, with a mean error of 10 %: the copies or half the
+// stream, whichever is longer, plus most of the stream (waves that share nothing overlap them badly), 0.3 ns per output of
+// the busiest CU, 2.2 us per million outputs, and the tiles' own packs (packUs); rows of any alignment take twice the
+// copies' time, and batches with a weight each (`weights`) stream all of A and B. f32: the estimate, which was within 8 %,
+// or nine tenths of it and 0.45 ns per output of the busiest CU. Of 20000 drawn layers 793 change sides against the
+// comparison of the bare estimates: 176 of them had been slower than the other kernel by 3 % and more (up to 1.5 times), 5
+// are now (up to 10 %); the 793 take 0.89 of the time.
+// Measured, against the other kernel: bf16 64 x 4096 x 4096 10 us (31), 64 x 11008 x 4096 22 (48), 192 x 4096 x 11008 45
+// (48), 400 x 4096 x 4096 27 (45), 16 batches of 32 x 1024 x 4096 33 (91); f16 x s8 4 x 4096 x 4096 6.1 (21.5), 128 x 4096 x
+// 4096 12 (55); u8 x s8 64 x 4096 x 4096 7.5 (47), 1024 x 4096 x 4096 40 (51). The others stay where a weight is wide for
+// its depth (bf16 255 x 14336 x 4096 55 against 47, 742 x 7968 x 256 34 against 22; f32 10925 x 2304 x 376 304 against 223)
+// and where the small tiles re-read A and B too often (M large; 64 batches of 128 x 512 x 2048 72 against 51).
+// 16-bit products of up to 16 rows have the decode kernels. Whole 256-row tiles of 16-bit products with whole k-tiles keep
+// the plans that tests of the dispatch name, although up to 32 tiles of 256 x 256 the wave-K tiles are the faster ones (256
+// x 4096 x 4096 23 against 38 us, 512 x 4096 x 4096 35 against 49; from 43 tiles on slower: 256 x 11008 x 4096 57 against
+// 50, 1024 x 4096 x 4096 65 against 51). Less than 4 whole k-tiles leave most waves without one. minParts (f32): the fewest
+// chains of 2-k steps that K is dealt to, for no longer chain of rounded sums than otherUs' kernel has: a wave's MFMAs are
+// of 2 k, with 16 rows or columns of 4. binary: the epilogue reads a second operand.
+inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, int64_t weights, int ct, bool weight8,
+                            bool kmajor, bool byRow, bool binary, double packUs, double otherUs, int minParts = 1)
 {
     struct Tile {
         int cfg, bm, bn, waves;
@@ -186,9 +201,12 @@ inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, in
         return 0;
     }
     const double mac = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K * batches);
-    const double stream = static_cast<double>(N) * static_cast<double>(K) * 128.0 / static_cast<double>(bk) / 6.6e6;
+    const double mn = static_cast<double>(M * N * batches) * 1e-6;
+    const double lineUs = static_cast<double>(K) * 128.0 / static_cast<double>(bk) / 6.6e6;  // a row of k at 6.6 TB/s
+    const double stream = static_cast<double>(N) * lineUs;
+    const double streamAll = static_cast<double>(N * weights + (weights > 1 ? M * batches : 0)) * lineUs;
     int best = 0;
-    double bestUs = 0.0;
+    double bestUs = 0.0, cost = 0.0;
     for (const Tile &t : kTiles) {
         if ((kmajor && t.bn < 64) || (t.bm == 16 && (M > 16 || (bk == 64 && !byRow))) ||
             (byRow && !kudnn_wavek_reg_tile(t.bm, t.bn, t.waves)) || t.waves * (t.bm == 16 || t.bn == 16 ? 2 : 1) < minParts) {
@@ -198,31 +216,42 @@ inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, in
         const double kb = (t.bm * (f16w8 ? 2 : 1) + t.bn) / 8.0;  // KB of a k-tile: a wave's stage
         const int64_t tiles = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn) * batches;
         const int64_t perCu = (tiles + 255) / 256, ktiles = (KT + waves - 1) / waves * waves;
-        const double copies = static_cast<double>(perCu * ktiles) * kb * t.nsPerKB * (byRow ? 1.15e-3 : (kmajor ? 1.08e-3 : 1e-3)) *
+        const double copies = static_cast<double>(perCu * ktiles) * kb * t.nsPerKB * 1e-3 *
                               (static_cast<double>(perCu * waves) * kb > 160.0 ? t.over : 1.0);
         const double mfma = f32 ? static_cast<double>(perCu * t.bm * t.bn) * 2e-6 * static_cast<double>(ktiles * bk) / t.f32Rate
                                 : mac * 2.0 / (ct == KUDNN_DT_S8 ? 1.4e9 : 0.8e9);
         // a part of the CUs streams a part of HBM's rate: in proportion for k-rows, less so for rows
-        const double part = tiles < 256 ? 256.0 / static_cast<double>(tiles) : 1.0;
-        const double hbm = stream * (kmajor ? part : std::sqrt(part));
-        const double busy = copies > mfma ? copies : mfma;
-        const double us = 4.2 + (busy > hbm ? busy + 0.15 * stream : hbm + 0.15 * copies);
+        double part = tiles < 256 ? 256.0 / static_cast<double>(tiles) : 1.0;
+        part = kmajor ? part : std::sqrt(part);
+        const double copyUs = copies * (byRow ? 1.15 : (kmajor ? 1.08 : 1.0)), busy = std::max(copyUs, mfma), hbm = stream * part;
+        const double us = 4.2 + (busy > hbm ? busy + 0.15 * stream : hbm + 0.15 * copyUs);
         if (best == 0 || us < bestUs) {
             best = t.cfg;
             bestUs = us;
+            const double out = static_cast<double>(perCu * t.bm * t.bn) * 1e-3;
+            if (f32) {
+                cost = std::max(us, 0.9 * us + 0.45 * out);
+            } else {
+                cost = 4.0 + std::max(0.9 * std::max(copies * (byRow ? 1.95 : 1.0), mfma), 0.58 * streamAll * part) +
+                       0.79 * streamAll + 0.31 * (t.cfg == KUDNN_CFG_WAVEK_64x64_W4 ? 0.63 : 1.0) * out +
+                       (binary ? 2.57 : 2.2) * mn + packUs;
+            }
         }
     }
-    return bestUs < otherUs ? best : 0;
+    return cost < otherUs ? best : 0;
 }
 
 // The same for batches of 16-bit products of at most 256 k (scores of attention heads, say), which spend their time on
 // tiles that start and end. One wave per 64 x 64 tile took 7 us + 2.5 ns a tile + 1 ns a k-tile of it; the ping-pong
 // kernel 3 us + 7.5 us a round of 256 tiles of 256 x 256, which ragged M and N leave partly empty, + 1.9 us a k-tile of
 // it; the 4-wave kernel 4 us + 4.2 us a round of 256 tiles of 128 x 128 + 0.9 us a k-tile. K off the k-tile adds two
-// packs to the last two. Up to 768 tiles, three a CU, four waves share one: 5.6-7 us a call against 7.6-9.2. Measured
-// (bf16, against the other kernel): 63 x (192 x 376 x 80) 31 -> 12 us, 32 x (256 x 256 x 96) 21 -> 7, 64 x (2048 x 128 x
-// 128) 32 -> 26, 20 x (300 x 1000 x 128) 15.4 -> 12.6; 32 x (1024 x 1024 x 128) stays: 44 against 27.
-inline int kudnn_wavek_batch_rule(int64_t M, int64_t N, int64_t K, int64_t batches, bool pingpong, double packUs)
+// packs to the last two. Up to 768 tiles, three a CU, four waves share one: 5.3 us + 2.5 ns a tile, or, with several tiles a
+// CU and short products, 4.5 us + 0.22 us a tile of the busiest CU + 0.4 us a k-tile of it + 1.4 us per million outputs. A
+// binary operand, which only the other kernels read ahead, adds to both. Measured (bf16, against the other kernel): 63 x
+// (192 x 376 x 80) 31 -> 12 us, 32 x (256 x 256 x 96) 21 -> 7, 64 x (2048 x 128 x 128) 32 -> 26, 20 x (300 x 1000 x 128)
+// 15.4 -> 12.6; these stay: 32 x (1024 x 1024 x 128) 44 against 27, 13 x (640 x 256 x 64) 10.2 against 7.9, 39 x (256 x 576
+// x 64) with an addend 19.5 against 14.8. Over 579 batches the side taken costs 1.2 % more than the better one.
+inline int kudnn_wavek_batch_rule(int64_t M, int64_t N, int64_t K, int64_t batches, bool pingpong, bool binary, double packUs)
 {
     const int64_t KT = (K + 63) / 64;
     if (batches < 2 || KT > 4) {
@@ -231,11 +260,13 @@ inline int kudnn_wavek_batch_rule(int64_t M, int64_t N, int64_t K, int64_t batch
     const int64_t bm = pingpong ? 256 : 128;
     const int64_t tiles = (M + 63) / 64 * ((N + 63) / 64) * batches;
     const double rounds = static_cast<double>(((M + bm - 1) / bm * ((N + bm - 1) / bm) * batches + 255) / 256);
-    const double kt = static_cast<double>(KT);
+    const double kt = static_cast<double>(KT), t = static_cast<double>(tiles), perCu = static_cast<double>((tiles + 255) / 256);
+    const double mn = static_cast<double>(M * N * batches) * 1e-6;
     const double other = packUs + (pingpong ? 3.0 + rounds * (7.5 + 1.9 * kt) : 4.0 + rounds * (4.2 + 0.9 * kt));
     const bool four = tiles <= 768;
-    const double us = four ? 5.3 + 2.5e-3 * static_cast<double>(tiles) : 7.0 + static_cast<double>(tiles) * (2.5e-3 + 1e-3 * kt);
-    return us < other ? (four ? KUDNN_CFG_WAVEK_64x64_W4 : KUDNN_CFG_WAVEK_64x64_W1) : 0;
+    const double us = four ? std::max(5.3 + 2.5e-3 * t, 4.5 + perCu * (0.22 + 0.4 * kt) + 1.4 * mn) : 7.0 + t * (2.5e-3 + 1e-3 * kt);
+    const double operand = binary ? (four ? 0.5 : 1.0) + 0.3 * mn : 0.0;
+    return us + operand < other ? (four ? KUDNN_CFG_WAVEK_64x64_W4 : KUDNN_CFG_WAVEK_64x64_W1) : 0;
 }
 int kudnn_launch_gemm_pingpong(const GemmOperands &op, const EpiParams &ep, int64_t batches, int ct, void *ws,
                                bool slicesOk, hipStream_t stream);

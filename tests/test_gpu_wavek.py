@@ -237,3 +237,48 @@ def test_planner_rule():
     assert "wavek" in plan8(1024, 16384, 4096, K.U8, K.S8, K.S32)
     assert plan32(107, 2176, 1984).startswith("mfma_f32_kslice_32x") and "_16x32" in plan32(240, 1298, 1400)
     assert plan32(128, 1024, 1024).startswith("mfma_f32_kslice_16x32") and plan32(2048, 4096, 4096).startswith("mfma_f32_128x128")
+
+
+def test_planner_leaves_what_the_other_kernels_do_faster():
+    # products that the estimates without outputs, batches and unaligned copies had moved to the wave-K tiles, measured (us)
+    # on those tiles and on the other kernel
+    def batch(B, M, Kd, N, wl="ACB", bin=K.BIN_NONE):
+        dy = K.desc([B, M, N], K.BF16)
+        return K.LinearPostOps(K.desc([B, M, Kd], K.BF16), K.desc([B, Kd, N], K.BF16, wl), dy, binary=bin,
+                               src=dy if bin else None).describe()
+
+    def one(M, Kd, N, adt=K.BF16, bdt=None, wl="BA", xl="AB"):
+        return K.Gemm(K.desc([M, Kd], adt, xl), K.desc([Kd, N], bdt or adt, wl), K.desc([M, N], adt)).describe()
+    other = [batch(64, 128, 2048, 512, "ABC"),      # 72, 51
+             batch(64, 128, 2048, 512),             # 71, 54
+             batch(32, 300, 512, 512),              # 28, 21
+             batch(64, 128, 512, 512),              # 30, 24
+             batch(13, 640, 64, 256),               # 10.2, 7.9
+             batch(39, 256, 64, 576, "ABC", K.BIN_ADD),  # 19.5, 14.8
+             one(742, 256, 7968, wl="AB"),          # 34, 22
+             one(4096, 512, 1024, K.F16, K.S8),     # 26, 23
+             one(10925, 376, 2304, K.F32),          # 304, 223
+             one(88640, 264, 256, K.F16, xl="BA"),  # 124, 95
+             one(2048, 2676, 1408),                 # 86, 70
+             one(693, 1222, 4936),                  # 55, 48
+             one(1, 16384, 4, K.F16, K.S8)]         # 9.8, 7.6
+    for d in other:
+        assert "wavek" not in d and "_w4" not in d and "percu" not in d, d
+    wavek = [batch(16, 32, 4096, 1024, "ABC"),      # 33, 91
+             batch(16, 17, 2048, 4096),             # 61, 80
+             batch(8, 17, 512, 2048),               # 7.3, 11.3
+             one(1216, 689, 3412, K.F16, wl="AB"),  # 35, 54
+             one(17, 4096, 3264, wl="AB"),          # 17.5, 30
+             one(1, 9600, 64, K.F16, K.S8)]         # 6.9, 12
+    for d in wavek:
+        assert "wavek" in d, d
+
+
+def test_planner_sixty_five_to_seventy_nine_tiles():
+    # one round of 128 x 128 tiles beats two K slices of 256 x 256 ones; two rounds do not. A weight stored [K][N] is read in
+    # place by the sliced kernel
+    def plan(M, Kd, N, wl="BA"):
+        return K.LinearPostOps(K.desc([M, Kd], K.BF16), K.desc([Kd, N], K.BF16, wl), K.desc([M, N], K.BF16)).describe()
+    assert plan(384, 4224, 8832).startswith("mfma_bf16_128x128 ")    # 49 us against 60
+    assert plan(800, 2688, 4352).startswith("mfma_bf16_128x128 ")    # 37 against 47
+    assert " kslices=2" in plan(738, 10112, 5896) and " kslices=2" in plan(800, 2688, 4352, "AB")
