@@ -65,17 +65,26 @@ int kudnn_pingpong_slice_tail(const GemmOperands &op, int64_t batches, int ct);
 constexpr int64_t KUDNN_FIXED_BYTES = int64_t(64) << 20, KUDNN_FIXED_COUNTERS = 512;
 constexpr int64_t KUDNN_FIXED_WORKSPACE = KUDNN_FIXED_BYTES - KUDNN_FIXED_COUNTERS;
 // Whether S slices leave every call of the allocation-free entry point accepted that is accepted unsliced: with no
-// operand packed, either or both (16-bit), what fits the scratch without the sums fits with them.
-inline bool kudnn_slices_fit(int64_t M, int64_t N, int64_t K, int64_t S)
+// operand packed, either or both (16-bit), what fits the scratch without the sums fits with them. `base`: the columns a row
+// of sums takes in the calls that have to stay accepted (0: no sums), `ld`: the ones it is to take.
+inline bool kudnn_slices_fit(int64_t M, int64_t N, int64_t K, int64_t S, int64_t base, int64_t ld)
 {
     const auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
-    const int64_t sums = up(S * M * ((N + 31) / 32 * 32) * 4), a = up(M * K * 2), b = up(N * K * 2);
+    const int64_t a = up(M * K * 2), b = up(N * K * 2), from = up(S * M * base * 4), to = up(S * M * ld * 4);
     for (const int64_t packs : {int64_t(0), a, b, a + b}) {
-        if (packs <= KUDNN_FIXED_WORKSPACE && packs + sums > KUDNN_FIXED_WORKSPACE) {
+        if (packs + from <= KUDNN_FIXED_WORKSPACE && packs + to > KUDNN_FIXED_WORKSPACE) {
             return false;
         }
     }
     return true;
+}
+// Columns that a row of the slices' sums takes: whole 128-byte lines (816 x 7048 x 4096 in two slices 103 -> 80 us) where
+// every call that fits the scratch with whole 32-byte chunks still fits it, else those (512 x 3073 x 6784 with a packed
+// weight needs 66.93 MB of 67.11 that way, 67.12 with lines).
+inline int64_t kudnn_slice_pitch(int64_t M, int64_t N, int64_t K, int64_t S)
+{
+    const int64_t lines = (N + 31) / 32 * 32, chunks = (N + 7) / 8 * 8;
+    return kudnn_slices_fit(M, N, K, S, chunks, lines) ? lines : chunks;
 }
 // The planner's K-slice count for the ping-pong kernel (0: none) of an M x N grid with KT k-tiles of 128 bytes.
 // Measured on MI355X over 26 shapes (M 256..4096, N 1152..14336, K 2048..14336, against the unsliced ping-pong, its
@@ -110,7 +119,7 @@ inline int kudnn_kslice_rule(int64_t M, int64_t N, int64_t KT, int64_t batches, 
         const double kt = static_cast<double>(KT), mn = static_cast<double>(M) * static_cast<double>(N);
         const double whole = 5.0 + (M % 256 != 0 ? 1.2 : 1.05) * kt;
         const double half = 9.0 + 0.6 * kt * (tiles > 96 ? 1.1 : 1.0) + mn * 16.0 / 3.6e6;
-        S = half * 1.05 < whole && kudnn_slices_fit(M, N, KT * 64, 2) ? 2 : 0;
+        S = half * 1.05 < whole && kudnn_slices_fit(M, N, KT * 64, 2, 0, (N + 31) / 32 * 32) ? 2 : 0;
     }
     return S >= 2 ? static_cast<int>(S) : 0;
 }

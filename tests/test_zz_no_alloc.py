@@ -120,3 +120,24 @@ def test_noalloc_refuses_slices_that_do_not_fit():
     plan.run(x, w, y)
     torch.cuda.synchronize()
     assert not bool(y.any()), "the allocating entry point did not run the plan"
+
+
+@pytest.mark.parametrize("M,N,Kd,xl,plan", [(512, 3073, 6784, "AB", "packB kslices=4"), (4096, 1160, 3520, "BA", "packA kmajorB kslices=2")])
+def test_noalloc_slices_beside_a_pack(M, N, Kd, xl, plan):
+    # sums and a pack that fill the scratch: 66.93 and 66.85 MB of 67.11 with rows of sums of whole 32-byte chunks, more than
+    # the scratch with rows of whole lines
+    x = torch.randn(M * Kd, device="cuda").bfloat16()
+    w = (torch.randn(N * Kd, device="cuda") * 0.03).bfloat16()
+    want, got = (torch.zeros(M * N, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    p = K.LinearPostOps(K.desc([M, Kd], K.BF16, xl), K.desc([Kd, N], K.BF16, "AB"), K.desc([M, N], K.BF16))
+    assert plan in p.describe(), p.describe()
+    p.run(x, w, want)
+    st = K.lib().kudnn_linear_postops_run_noalloc(p.handle, x.data_ptr(), w.data_ptr(), got.data_ptr(), None, None,
+                                                  ctypes.c_float(1.0), torch.cuda.current_stream().cuda_stream)
+    assert st == K.SUCCESS, K.last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    a = x.view(Kd, M).t() if xl == "BA" else x.view(M, Kd)
+    rows = torch.arange(0, M, 37, device="cuda")  # a few rows in f32: sums of Kd products of bf16 numbers, rounded once
+    ref = a[rows].float().contiguous() @ w.view(Kd, N).float()
+    assert float((want.view(M, N)[rows].float() - ref).norm() / ref.norm()) < 2.0 ** -8
