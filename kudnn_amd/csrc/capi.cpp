@@ -399,7 +399,7 @@ int DispatchDt(const kudnn_tensor_desc &d, int nd)
 // fold too; their batch strides are updated with the core's.
 int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudnn_tensor_desc &c,
               const kudnn_tensor_desc *bias, GemmCore &core, const char *op, TensorSpec *extra0 = nullptr,
-              TensorSpec *extra1 = nullptr)
+              TensorSpec *extra1 = nullptr, bool fixedScratch = false)
 {
     TensorSpec *extras[2] = {extra0, extra1};
     const int nd = a.ndims;
@@ -570,16 +570,51 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
                                        core.B.bs[1] % 8 == 0 && core.B.bs[2] % 8 == 0 && core.N % 8 == 0 &&
                                        !std::getenv("KUDNN_HIP_PACK_KMAJOR"));
     const bool weight8 = w8 && (chunkedAB || byRow);
+    // ... and what it still has to pack
+    const bool packAWk = !(chunkedAB || byRow) && (kmajorWk ? !chunked(core.A) : core.A.staticPack);
+    const bool packBWk = !(chunkedAB || byRow) && !kmajorWk && core.B.staticPack;
 
     // engine and tile configuration
     const int64_t batches = core.Batches();
+    // Whether a plan of the allocation-free entry point (`fixedScratch`) fits its scratch with the kernel of core.cfg wherever
+    // it does on the wave-K tiles, which need no sums and fewer packs, for bases on and off 16 bytes. Where it does not, the
+    // comparison of the bare estimates may give the product to those tiles too: such calls have been accepted.
+    const auto fitsScratch = [&](bool bInPlace) {
+        if (!fixedScratch) {
+            return true;
+        }
+        GemmOperands shape{};
+        shape.M = core.M;
+        shape.N = core.N;
+        shape.K = core.kp;
+        const auto bytes = [&](const OperandSpec &o) {
+            const int64_t copies = o.bs[0] == 0 && o.bs[1] == 0 && o.bs[2] == 0 ? 1 : batches;
+            return (copies * o.rows * core.kp * DtSize(core.computeDt) + 255) / 256 * 256;
+        };
+        const int64_t a = bytes(core.A), b = bytes(core.B);
+        int64_t sums = static_cast<int64_t>(core.cfg == KUDNN_CFG_BF16_PINGPONG_256x256
+                                                ? kudnn_pingpong_workspace_bytes(shape, batches, core.computeDt, true)
+                                                : kudnn_gemm_workspace_bytes(shape, batches, core.cfg, core.computeDt));
+        sums = (sums + 255) / 256 * 256;
+        if (core.computeDt == KUDNN_DT_S8) {
+            sums += (batches * (core.M + core.N) * 4 + 511) / 256 * 256;  // row sums of a u8 operand's partner
+        }
+        for (int off = 0; off < 4; ++off) {
+            const int64_t here = (core.A.staticPack || off & 1 ? a : 0) + ((core.B.staticPack && !bInPlace) || off & 2 ? b : 0);
+            const int64_t wk = (packAWk || off & 1 ? a : 0) + (packBWk || off & 2 ? b : 0);
+            if (wk <= KUDNN_FIXED_WORKSPACE && here + sums > KUDNN_FIXED_WORKSPACE) {
+                return false;
+            }
+        }
+        return true;
+    };
     int64_t weights = 1;  // distinct weights of the batches
     for (int d = 0; d < 3; ++d) {
         weights *= core.B.bs[d] != 0 ? core.bdim[d] : 1;
     }
     const double mbAB = (static_cast<double>(batches * core.M * core.K * DtSize(core.A.dt)) +
                          static_cast<double>(weights * core.N * core.K * DtSize(core.B.dt))) * 1e-6;
-    bool tailSplit = false;
+    bool tailSplit = false, oneRound = false;
     if (core.computeDt != KUDNN_DT_F32) {
         if (core.M <= 16 && lowp16) {
             core.engine = ENGINE_SKINNY_BF16;
@@ -622,9 +657,9 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
             // 128 x 128 tiles stay sliced (738 x 5896 x 10112).
             const double mn = static_cast<double>(core.M * core.N) * 1e-6, ktd = static_cast<double>(kt);
             const int64_t t128 = (core.M + 127) / 128 * ((core.N + 127) / 128) * batches;
-            const bool oneRound = t256 > 64 && t256 < 80 && 4.0 + static_cast<double>((t128 + 255) / 256) * (5.6 + 0.63 * ktd) <
-                                                               11.8 + 0.52 * ktd + 3.7 * mn;
-            const bool fourWave = batches == 1 && core.B.s_r != 1 && ((t256 >= 32 && t256 <= 64 && kt <= 64) || oneRound);
+            oneRound = batches == 1 && core.B.s_r != 1 && t256 > 64 && t256 < 80 &&
+                       4.0 + static_cast<double>((t128 + 255) / 256) * (5.6 + 0.63 * ktd) < 11.8 + 0.52 * ktd + 3.7 * mn;
+            const bool fourWave = (batches == 1 && core.B.s_r != 1 && t256 >= 32 && t256 <= 64 && kt <= 64) || oneRound;
             core.cfg = (t256 >= 80 || tailSplit || slices) && !fourWave ? KUDNN_CFG_BF16_PINGPONG_256x256
                                                                         : KUDNN_CFG_BF16_128x128;
         }
@@ -661,11 +696,18 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         }
         other += s8 && core.A.dt == KUDNN_DT_U8 ? 10.7 + 0.44 * mbAB
                                                 : (packsO == 2 ? 9.4 + 0.3 * mbAB : (packsO == 1 ? 2.4 + 0.27 * mbAB : 0.0));
-        // what the wave-K tiles themselves have to pack
-        const int packsW = chunkedAB || byRow ? 0
-                           : kmajorWk         ? (chunked(core.A) ? 0 : 1)
-                                              : (core.A.staticPack ? 1 : 0) + (core.B.staticPack ? 1 : 0);
+        const int packsW = (packAWk ? 1 : 0) + (packBWk ? 1 : 0);
         const double packUs = packsW == 2 ? 2.8 + 0.21 * mbAB : (packsW == 1 ? 5.4 + 0.06 * mbAB : 0.0);
+        const bool fits = fitsScratch(bInPlace);
+        double bare = 0.0;
+        if (!fits) {
+            const double nk = static_cast<double>(core.N * core.K);
+            bare = !pingpong && !(oneRound && S >= 2) ? (other < 1e30 ? r128 * (4.0 + (s8 ? 0.72 : 0.66) * kt) : other)
+                             : (S >= 2 ? 9.0 + 1.2 * kt / S + S * mn * 8.0 / 3.6 : 5.0 + 1.15 * kt * r256);
+            bare += weight8 ? 3.0 + nk * 0.75e-6
+                            : (s8 && core.A.dt == KUDNN_DT_U8 ? 14.0 + nk * 0.47e-6
+                                                              : (byRow || core.K % bk != 0 ? 5.0 + mbAB * 2.0 / 4.2 : 0.0));
+        }
         // an integer product with a u8 weight needs row sums of A, and an 8-bit weight of an f16 product that cannot be
         // read in place is packed to f16: both stay with the other kernels. A weight of at most 16 rows is one workgroup's
         // work there, of 8 chains of k-tiles; the row kernel with its pack is the faster one for a deep K (f16 x s8
@@ -674,7 +716,7 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         if (!(s8 && tailSplit && t256 == 64 && core.A.dt == KUDNN_DT_S8) && (core.B.dt != KUDNN_DT_U8 || weight8) &&
             (core.M > 16 || !lowp16 || weight8 || byRow) && !fewRows) {
             if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, weights, core.computeDt, weight8,
-                                                kmajorWk, byRow, binary, packUs, other)) {
+                                                kmajorWk, byRow, binary, packUs, other, bare)) {
                 core.engine = ENGINE_MFMA_BF16;
                 core.cfg = wk;
             }
@@ -682,7 +724,8 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         if (lowp16 && core.M > 16 && core.B.dt == core.computeDt && (chunkedAB || (kmajorWk && chunked(core.A))) &&
             !kudnn_is_wavek(core.cfg)) {
             const double packsOther = core.K % 64 != 0 ? 5.0 + mbAB * 2.0 / 4.2 : 0.0;
-            if (const int wk = kudnn_wavek_batch_rule(core.M, core.N, core.K, batches, pingpong, binary, packsOther)) {
+            if (const int wk = kudnn_wavek_batch_rule(core.M, core.N, core.K, batches, pingpong, binary, packsOther,
+                                                      !fits)) {
                 core.cfg = wk;
             }
         }
@@ -731,7 +774,7 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
             }
             other += core.K % bk != 0 ? 5.0 + mbAB * 2.0 / 4.2 : 0.0;
             if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, weights, core.computeDt, false, false,
-                                                byRow, false, 0.0, other, parts)) {
+                                                byRow, false, 0.0, other, fitsScratch(false) ? 0.0 : other, parts)) {
                 core.engine = ENGINE_MFMA_BF16;
                 core.cfg = wk;
             }
@@ -2065,7 +2108,7 @@ int kudnn_linear_postops_create(const kudnn_tensor_desc *a, const kudnn_tensor_d
         p->x.hasSrc = true;
         p->x.Src = SpecOf(*src);
     }
-    s = BuildCore(*a, *b, *y, &p->bias, p->core, "LinearPostOpsFWD", p->x.hasSrc ? &p->x.Src : nullptr);
+    s = BuildCore(*a, *b, *y, &p->bias, p->core, "LinearPostOpsFWD", p->x.hasSrc ? &p->x.Src : nullptr, nullptr, true);
     if (s == KUDNN_STATUS_SUCCESS && !IsFp(y->dtype) && (act_kind != KUDNN_ACT_UNIMPLEMENTED || p->x.hasSrc)) {
         s = Fail(KUDNN_STATUS_UNSUPPORTED, "LinearPostOpsFWD: a Linear into an integer output takes no activation or "
                                            "binary operand");

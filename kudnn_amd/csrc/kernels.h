@@ -189,9 +189,11 @@ int kudnn_launch_gemm_wavek8(const GemmOperands &op, const EpiParams &ep, int64_
 // x 4096 x 4096 23 against 38 us, 512 x 4096 x 4096 35 against 49; from 43 tiles on slower: 256 x 11008 x 4096 57 against
 // 50, 1024 x 4096 x 4096 65 against 51). Less than 4 whole k-tiles leave most waves without one. minParts (f32): the fewest
 // chains of 2-k steps that K is dealt to, for no longer chain of rounded sums than otherUs' kernel has: a wave's MFMAs are
-// of 2 k, with 16 rows or columns of 4. binary: the epilogue reads a second operand.
+// of 2 k, with 16 rows or columns of 4. binary: the epilogue reads a second operand. bareUs: the other kernel's estimate for
+// the comparison of the bare estimates, 0 where it does not count.
 inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, int64_t weights, int ct, bool weight8,
-                            bool kmajor, bool byRow, bool binary, double packUs, double otherUs, int minParts = 1)
+                            bool kmajor, bool byRow, bool binary, double packUs, double otherUs, double bareUs,
+                            int minParts = 1)
 {
     struct Tile {
         int cfg, bm, bn, waves;
@@ -247,7 +249,7 @@ inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, in
             }
         }
     }
-    return cost < otherUs ? best : 0;
+    return cost < otherUs || bestUs < bareUs ? best : 0;
 }
 
 // The same for batches of 16-bit products of at most 256 k (scores of attention heads, say), which spend their time on
@@ -259,8 +261,10 @@ inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, in
 // binary operand, which only the other kernels read ahead, adds to both. Measured (bf16, against the other kernel): 63 x
 // (192 x 376 x 80) 31 -> 12 us, 32 x (256 x 256 x 96) 21 -> 7, 64 x (2048 x 128 x 128) 32 -> 26, 20 x (300 x 1000 x 128)
 // 15.4 -> 12.6; these stay: 32 x (1024 x 1024 x 128) 44 against 27, 13 x (640 x 256 x 64) 10.2 against 7.9, 39 x (256 x 576
-// x 64) with an addend 19.5 against 14.8. Over 579 batches the side taken costs 1.2 % more than the better one.
-inline int kudnn_wavek_batch_rule(int64_t M, int64_t N, int64_t K, int64_t batches, bool pingpong, bool binary, double packUs)
+// x 64) with an addend 19.5 against 14.8. Over 579 batches the side taken costs 1.2 % more than the better one. bare: the
+// comparison without the several tiles' and the operand's terms.
+inline int kudnn_wavek_batch_rule(int64_t M, int64_t N, int64_t K, int64_t batches, bool pingpong, bool binary, double packUs,
+                                  bool bare)
 {
     const int64_t KT = (K + 63) / 64;
     if (batches < 2 || KT > 4) {
@@ -273,9 +277,12 @@ inline int kudnn_wavek_batch_rule(int64_t M, int64_t N, int64_t K, int64_t batch
     const double mn = static_cast<double>(M * N * batches) * 1e-6;
     const double other = packUs + (pingpong ? 3.0 + rounds * (7.5 + 1.9 * kt) : 4.0 + rounds * (4.2 + 0.9 * kt));
     const bool four = tiles <= 768;
-    const double us = four ? std::max(5.3 + 2.5e-3 * t, 4.5 + perCu * (0.22 + 0.4 * kt) + 1.4 * mn) : 7.0 + t * (2.5e-3 + 1e-3 * kt);
-    const double operand = binary ? (four ? 0.5 : 1.0) + 0.3 * mn : 0.0;
-    return us + operand < other ? (four ? KUDNN_CFG_WAVEK_64x64_W4 : KUDNN_CFG_WAVEK_64x64_W1) : 0;
+    double us = four ? 5.3 + 2.5e-3 * t : 7.0 + t * (2.5e-3 + 1e-3 * kt);
+    if (!bare) {
+        us = four ? std::max(us, 4.5 + perCu * (0.22 + 0.4 * kt) + 1.4 * mn) : us;
+        us += binary ? (four ? 0.5 : 1.0) + 0.3 * mn : 0.0;
+    }
+    return us < other ? (four ? KUDNN_CFG_WAVEK_64x64_W4 : KUDNN_CFG_WAVEK_64x64_W1) : 0;
 }
 int kudnn_launch_gemm_pingpong(const GemmOperands &op, const EpiParams &ep, int64_t batches, int ct, void *ws,
                                bool slicesOk, hipStream_t stream);

@@ -1,6 +1,8 @@
 """The wave-K kernel (small tiles whose K is dealt to the workgroup's waves): every tile at the edges of M, N and K, both
 weight layouts, batches, graph replay and the planner's choices, against the oracle. Integer-valued inputs make the f32
 sums exact in any order, so the comparisons are bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -282,3 +284,27 @@ def test_planner_sixty_five_to_seventy_nine_tiles():
     assert plan(384, 4224, 8832).startswith("mfma_bf16_128x128 ")    # 49 us against 60
     assert plan(800, 2688, 4352).startswith("mfma_bf16_128x128 ")    # 37 against 47
     assert " kslices=2" in plan(738, 10112, 5896) and " kslices=2" in plan(800, 2688, 4352, "AB")
+
+
+def test_planner_keeps_the_fixed_scratch_calls():
+    # plans of the allocation-free entry point: where the other kernel, the faster one, needs more than its scratch for packs
+    # and sums and the wave-K tiles do not, these keep the product; the other entry points go by time alone
+    for M, Kd, N, dt in ((448, 9898, 3808, K.F16), (744, 7776, 5888, K.BF16), (144, 9833, 8448, K.BF16)):
+        d = K.desc([M, Kd], dt), K.desc([Kd, N], dt, "BA"), K.desc([M, N], dt)
+        post, gemm = K.LinearPostOps(*d).describe(), K.Gemm(*d).describe()
+        assert "wavek" in post and "pack" not in post, post
+        assert "pingpong" in gemm and "packA packB kslices=" in gemm, gemm
+
+
+@pytest.mark.gpu
+def test_fixed_scratch_call_beside_a_large_pack(gpu):
+    M, Kd, N = 448, 9898, 3808
+    x, w = torch.randn(M, Kd, device="cuda").half(), (torch.randn(N, Kd, device="cuda") * 0.02).half()
+    y, z = (torch.zeros(M, N, device="cuda", dtype=torch.float16) for _ in range(2))
+    p = K.LinearPostOps(K.desc([M, Kd], K.F16), K.desc([Kd, N], K.F16, "BA"), K.desc([M, N], K.F16))
+    p.run(x, w, y)
+    st = K.lib().kudnn_linear_postops_run_noalloc(p.handle, x.data_ptr(), w.data_ptr(), z.data_ptr(), None, None,
+                                                  ctypes.c_float(1.0), torch.cuda.current_stream().cuda_stream)
+    assert st == K.SUCCESS, K.last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(y, z)
