@@ -3,9 +3,9 @@
 //
 // Computes Y = epilogue(A[M][K] x B[N][K]^T) as the 4-wave kernel does (gemm_mfma.hip), for products whose M is a few
 // tens to a few hundred rows: their time is the weight's way from HBM, and a chain of k-tiles with a barrier each
-// (copies issued, waited for, read, multiplied, one after the other by all waves of a tile) spent 650 cycles a k-tile
-// on it, whatever the depth of its ring; splitting K over workgroups instead cost 6 us a call for the exchange of the
-// sums. Here nothing in the K loop is shared:
+// (copies issued, waited for, read, multiplied, one after the other by all waves of a tile) holds it up: bf16 64 x 4096
+// x 4096, weights from HBM, 43.3 us a call on 128 x 128 tiles and 30.8 with K in four slices over workgroups, whose
+// sums meet in a second launch, against 14.5 here; 64 x 11008 x 4096 45.2 against 28.2. Nothing in the K loop is shared:
 //  - Wave w of W takes k-tiles w, w + W, w + 2 W, ... (128 bytes of each weight row) and accumulates the whole tile over
 //    them. It owns a stage of LDS for one k-tile of A and B; it waits for its own copies (vmcnt), reads all fragments
 //    into registers, issues the copies of its next k-tile into the same stage, and runs the MFMAs while they fly. No
@@ -15,9 +15,11 @@
 //  - K needs no padding to whole k-tiles: a copy of the last k-tile reads zeros for the 16-byte chunks past K. Rows that
 //    are no multiple of 16 bytes apart, or end inside a chunk, go through registers instead of the LDS DMA (REG): loads
 //    at any element alignment, written to the stage once the previous k-tile's fragments are out of it.
-// What bounds it: the bytes that pass a CU's address unit, (BM + BN) x 128 per k-tile at about 22 cycles per KB, and
-// the bytes of weight in flight over the whole chip against HBM's latency. So a tile is small where the grid is small,
-// and the narrow ones (BN = 16, on 16 x 16 MFMAs) give N = 4096 a workgroup per CU.
+// What bounds it, by counters: the bytes of weight in flight over the whole chip against HBM's latency where calls are
+// small (64 x 4096 x 4096: waves wait 0.72 of their cycles), and from 64 x 11008 x 4096 up as much the copies through a
+// CU's address unit, (BM + BN) x 128 bytes per k-tile at 21 to 27 of its cycles per KB (busy 0.4 to 0.7 of the time; the
+// MFMAs are busy 0.3 at most). So a tile is small where the grid is small, and the narrow ones (BN = 16, on 16 x 16
+// MFMAs) give N = 4096 a workgroup per CU.
 // A 16-bit weight stored [K][N] is read in place by the tiles of BN >= 64 (KM): a k-tile of B is then 64 k-rows of whole
 // 128-byte lines, and gfx950's transposing LDS read hands each lane 4 consecutive k of one n.
 // An 8-bit weight of an f16 product stays 8-bit up to the registers: a k-tile is then 128 k (two 128-byte pieces of an A
@@ -152,7 +154,8 @@ __global__ __launch_bounds__(W * 64, 1) void gemm_wavek_kernel(GemmOperands op, 
     constexpr int GA = BM / 8, GB = BN / 8;       // 1 KB copies of a k-tile (A: per piece)
     constexpr int kStage = (BM * AH + BN) * kChunks;  // uint4 per wave
     static_assert(!KM || (BN >= 64 && !INT && !B8 && !F32 && !REG), "K-major B: 16-bit elements, whole lines of columns");
-    // K-major B: a copy covers kRpc k-rows of a segment of kSegN columns (128 bytes of a k-row)
+    // K-major B: a copy covers kRpc k-rows of a segment of kSegN columns (128 bytes of a k-row). kSeg: segments of the tile;
+    // narrower tiles have no K-major form, and only a divisor's value
     constexpr int kSegN = 64, kSeg = BN < 64 ? 1 : BN / kSegN, kRpc = 8, kRowC = 8;
     // blocks of columns whose sums are exchanged at a time: the most that fit a wave's stage
     constexpr int JP = BM * BN * 4 <= kStage * 16 ? FN : (BM * BN * 2 <= kStage * 16 ? FN / 2 : 1);
@@ -539,6 +542,8 @@ int launch_type(const GemmOperands &op, const EpiParams &ep, int64_t batches, in
         case KUDNN_CFG_WAVEK_32x16: return launch_tile<CT, BT, 32, 16, 8>(op, ep, batches, reg, stream);
         case KUDNN_CFG_WAVEK_32x32: return launch_tile<CT, BT, 32, 32, 8>(op, ep, batches, reg, stream);
         case KUDNN_CFG_WAVEK_32x64: return launch_tile<CT, BT, 32, 64, 6>(op, ep, batches, reg, stream);
+        // 6 waves of f16 with 8-bit weights spill a register or two in one form each: 64 x 32 with rows of any alignment
+        // 12 bytes a lane, 64 x 64 in whole chunks 8; outside those forms no instance spills
         case KUDNN_CFG_WAVEK_64x32: return launch_tile<CT, BT, 64, 32, 6>(op, ep, batches, reg, stream);
         case KUDNN_CFG_WAVEK_64x64: return launch_tile<CT, BT, 64, 64, f16w8 ? 6 : 8>(op, ep, batches, reg, stream);
         case KUDNN_CFG_WAVEK_64x64_W4: return launch_tile<CT, BT, 64, 64, f16w8 ? 3 : 4>(op, ep, batches, reg, stream);
