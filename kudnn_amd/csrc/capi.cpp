@@ -723,9 +723,18 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         }
         if (lowp16 && core.M > 16 && core.B.dt == core.computeDt && (chunkedAB || (kmajorWk && chunked(core.A))) &&
             !kudnn_is_wavek(core.cfg)) {
-            const double packsOther = core.K % 64 != 0 ? 5.0 + mbAB * 2.0 / 4.2 : 0.0;
+            // The 4-wave kernel packs a weight stored [K][N], which four waves a tile (up to 768 tiles) read in place: 57 x
+            // (192 x 128 x 192) 14.3 us with the pack, 11.7 without, 39 x (145 x 128 x 312) 16.2 and 12.3. Rows of no whole
+            // 16-byte runs lengthen every kernel's epilogue, the others' by more than the terms that the plain comparison
+            // of four waves a tile leaves out: 8 x (185 x 64 x 1487) 21.7 against 14.5; one wave a tile does not gain (50 x
+            // (512 x 128 x 541) 71 us on the ping-pong kernel, 100 on those tiles).
+            const bool four = (core.M + 63) / 64 * ((core.N + 63) / 64) * batches <= 768;
+            const double packsOther =
+                core.K % 64 != 0 ? 5.0 + mbAB * 2.0 / 4.2
+                                 : (kmajorWk && !pingpong && four
+                                        ? 3.0 + 0.75e-6 * static_cast<double>(weights * core.N * core.K * DtSize(core.B.dt)) : 0.0);
             if (const int wk = kudnn_wavek_batch_rule(core.M, core.N, core.K, batches, pingpong, binary, packsOther,
-                                                      !fits)) {
+                                                      !fits || (four && core.N % 8 != 0))) {
                 core.cfg = wk;
             }
         }

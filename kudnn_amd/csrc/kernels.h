@@ -255,13 +255,13 @@ inline int kudnn_wavek_rule(int64_t M, int64_t N, int64_t K, int64_t batches, in
 // The same for batches of 16-bit products of at most 256 k (scores of attention heads, say), which spend their time on
 // tiles that start and end. One wave per 64 x 64 tile took 7 us + 2.5 ns a tile + 1 ns a k-tile of it; the ping-pong
 // kernel 3 us + 7.5 us a round of 256 tiles of 256 x 256, which ragged M and N leave partly empty, + 1.9 us a k-tile of
-// it; the 4-wave kernel 4 us + 4.2 us a round of 256 tiles of 128 x 128 + 0.9 us a k-tile. K off the k-tile adds two
-// packs to the last two. Up to 768 tiles, three a CU, four waves share one: 5.3 us + 2.5 ns a tile, or, with several tiles a
-// CU and short products, 4.5 us + 0.22 us a tile of the busiest CU + 0.4 us a k-tile of it + 1.4 us per million outputs. A
-// binary operand, which only the other kernels read ahead, adds to both. Measured (bf16, against the other kernel): 63 x
+// it; the 4-wave kernel 4 us + 4.2 us a round of 256 tiles of 128 x 128 + 0.9 us a k-tile. packUs: what these two pack on
+// each call. Up to 768 tiles, three a CU, four waves share one: 5.3 us + 2.5 ns a tile, or, with several tiles a CU and
+// short products, 4.5 us + 0.22 us a tile of the busiest CU + 0.4 us a k-tile of it + 1.4 us per million outputs. A binary
+// operand, which only the other kernels read ahead, adds to both. Measured (bf16, against the other kernel): 63 x
 // (192 x 376 x 80) 31 -> 12 us, 32 x (256 x 256 x 96) 21 -> 7, 64 x (2048 x 128 x 128) 32 -> 26, 20 x (300 x 1000 x 128)
 // 15.4 -> 12.6; these stay: 32 x (1024 x 1024 x 128) 44 against 27, 13 x (640 x 256 x 64) 10.2 against 7.9, 39 x (256 x 576
-// x 64) with an addend 19.5 against 14.8. Over 579 batches the side taken costs 1.2 % more than the better one. bare: the
+// x 64) with an addend 19.5 against 14.8. Over 579 batches the side taken costs 1.1 % more than the better one. bare: the
 // comparison without the several tiles' and the operand's terms.
 inline int kudnn_wavek_batch_rule(int64_t M, int64_t N, int64_t K, int64_t batches, bool pingpong, bool binary, double packUs,
                                   bool bare)

@@ -271,6 +271,8 @@ def test_planner_leaves_what_the_other_kernels_do_faster():
              batch(64, 128, 512, 512),              # 30, 24
              batch(13, 640, 64, 256),               # 10.2, 7.9
              batch(39, 256, 64, 576, "ABC", K.BIN_ADD),  # 19.5, 14.8
+             batch(35, 256, 128, 256),              # 11.4, 8.9
+             batch(50, 512, 128, 541, bin=K.BIN_ADD),  # 100, 71
              one(742, 256, 7968, wl="AB"),          # 34, 22
              one(4096, 512, 1024, K.F16, K.S8),     # 26, 23
              one(10925, 376, 2304, K.F32),          # 304, 223
@@ -283,6 +285,9 @@ def test_planner_leaves_what_the_other_kernels_do_faster():
     wavek = [batch(16, 32, 4096, 1024, "ABC"),      # 33, 91
              batch(16, 17, 2048, 4096),             # 61, 80
              batch(8, 17, 512, 2048),               # 7.3, 11.3
+             batch(57, 192, 128, 192, "ABC"),       # 11.7, 14.3 with the weight's pack
+             batch(39, 145, 128, 312, "ABC"),       # 12.3, 16.2
+             batch(8, 185, 64, 1487),               # 14.5, 21.7: rows of no whole 16-byte runs
              one(1216, 689, 3412, K.F16, wl="AB"),  # 35, 54
              one(17, 4096, 3264, wl="AB"),          # 17.5, 30
              one(1, 9600, 64, K.F16, K.S8)]         # 6.9, 12
