@@ -699,15 +699,17 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         const int packsW = (packAWk ? 1 : 0) + (packBWk ? 1 : 0);
         const double packUs = packsW == 2 ? 2.8 + 0.21 * mbAB : (packsW == 1 ? 5.4 + 0.06 * mbAB : 0.0);
         const bool fits = fitsScratch(bInPlace);
-        double bare = 0.0;
-        if (!fits) {
-            const double nk = static_cast<double>(core.N * core.K);
-            bare = !pingpong && !(oneRound && S >= 2) ? (other < 1e30 ? r128 * (4.0 + (s8 ? 0.72 : 0.66) * kt) : other)
-                             : (S >= 2 ? 9.0 + 1.2 * kt / S + S * mn * 8.0 / 3.6 : 5.0 + 1.15 * kt * r256);
-            bare += weight8 ? 3.0 + nk * 0.75e-6
-                            : (s8 && core.A.dt == KUDNN_DT_U8 ? 14.0 + nk * 0.47e-6
-                                                              : (byRow || core.K % bk != 0 ? 5.0 + mbAB * 2.0 / 4.2 : 0.0));
-        }
+        const double nk = static_cast<double>(core.N * core.K);
+        double bareOther = !pingpong && !(oneRound && S >= 2) ? (other < 1e30 ? r128 * (4.0 + (s8 ? 0.72 : 0.66) * kt) : other)
+                           : (S >= 2 ? 9.0 + 1.2 * kt / S + S * mn * 8.0 / 3.6 : 5.0 + 1.15 * kt * r256);
+        bareOther += weight8 ? 3.0 + nk * 0.75e-6
+                             : (s8 && core.A.dt == KUDNN_DT_U8 ? 14.0 + nk * 0.47e-6
+                                                               : (byRow || core.K % bk != 0 ? 5.0 + mbAB * 2.0 / 4.2 : 0.0));
+        const double bare = fits ? 0.0 : bareOther;
+        // u8 x s8 on the ping-pong kernel moves only where the bare estimates say so too: with a long K the fit is a tenth
+        // high and the wave-K tiles' cost a quarter low (5748 x 1152 x 15168 191 us, 262 on those tiles; 67 of 91 such
+        // products were slower there, by 1.10 over all)
+        const bool agree = s8 && pingpong && core.A.dt == KUDNN_DT_U8;
         // an integer product with a u8 weight needs row sums of A, and an 8-bit weight of an f16 product that cannot be
         // read in place is packed to f16: both stay with the other kernels. A weight of at most 16 rows is one workgroup's
         // work there, of 8 chains of k-tiles; the row kernel with its pack is the faster one for a deep K (f16 x s8
@@ -715,8 +717,11 @@ int BuildCore(const kudnn_tensor_desc &a, const kudnn_tensor_desc &b, const kudn
         const bool fewRows = weight8 && core.M <= 2 && core.N <= 16 && core.K >= 12288 && batches == 1;
         if (!(s8 && tailSplit && t256 == 64 && core.A.dt == KUDNN_DT_S8) && (core.B.dt != KUDNN_DT_U8 || weight8) &&
             (core.M > 16 || !lowp16 || weight8 || byRow) && !fewRows) {
-            if (const int wk = kudnn_wavek_rule(core.M, core.N, core.K, batches, weights, core.computeDt, weight8,
-                                                kmajorWk, byRow, binary, packUs, other, bare)) {
+            const auto rule = [&](double otherUs, double bareUs) {
+                return kudnn_wavek_rule(core.M, core.N, core.K, batches, weights, core.computeDt, weight8, kmajorWk, byRow,
+                                        binary, packUs, otherUs, bareUs);
+            };
+            if (const int wk = !agree || rule(0.0, bareOther) ? rule(other, bare) : 0) {
                 core.engine = ENGINE_MFMA_BF16;
                 core.cfg = wk;
             }

@@ -263,8 +263,8 @@ def test_planner_leaves_what_the_other_kernels_do_faster():
         return K.LinearPostOps(K.desc([B, M, Kd], K.BF16), K.desc([B, Kd, N], K.BF16, wl), dy, binary=bin,
                                src=dy if bin else None).describe()
 
-    def one(M, Kd, N, adt=K.BF16, bdt=None, wl="BA", xl="AB"):
-        return K.Gemm(K.desc([M, Kd], adt, xl), K.desc([Kd, N], bdt or adt, wl), K.desc([M, N], adt)).describe()
+    def one(M, Kd, N, adt=K.BF16, bdt=None, wl="BA", xl="AB", ydt=None):
+        return K.Gemm(K.desc([M, Kd], adt, xl), K.desc([Kd, N], bdt or adt, wl), K.desc([M, N], ydt or adt)).describe()
     other = [batch(64, 128, 2048, 512, "ABC"),      # 72, 51
              batch(64, 128, 2048, 512),             # 71, 54
              batch(32, 300, 512, 512),              # 28, 21
@@ -279,7 +279,9 @@ def test_planner_leaves_what_the_other_kernels_do_faster():
              one(88640, 264, 256, K.F16, xl="BA"),  # 124, 95
              one(2048, 2676, 1408),                 # 86, 70
              one(693, 1222, 4936),                  # 55, 48
-             one(1, 16384, 4, K.F16, K.S8)]         # 9.8, 7.6
+             one(1, 16384, 4, K.F16, K.S8),         # 9.8, 7.6
+             one(5748, 15168, 1152, K.U8, K.S8, ydt=K.S32),   # 262, 191
+             one(1792, 11712, 4096, K.U8, K.S8, ydt=K.S32)]   # 201, 148
     for d in other:
         assert "wavek" not in d, d
     wavek = [batch(16, 32, 4096, 1024, "ABC"),      # 33, 91
@@ -290,6 +292,7 @@ def test_planner_leaves_what_the_other_kernels_do_faster():
              batch(8, 185, 64, 1487),               # 14.5, 21.7: rows of no whole 16-byte runs
              one(1216, 689, 3412, K.F16, wl="AB"),  # 35, 54
              one(17, 4096, 3264, wl="AB"),          # 17.5, 30
+             one(1024, 4096, 4096, K.U8, K.S8, ydt=K.S32),    # 41, 83
              one(1, 9600, 64, K.F16, K.S8)]         # 6.9, 12
     for d in wavek:
         assert "wavek" in d, d
